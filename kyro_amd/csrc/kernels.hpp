@@ -18,7 +18,7 @@ enum ErrorBits : int {
 };
 
 
-enum AttnKernel : int { ATTN_KERNEL_VECTOR = 1, ATTN_KERNEL_MFMA = 2 };
+enum AttnKernel : int { ATTN_KERNEL_VECTOR = 1, ATTN_KERNEL_MFMA = 2, ATTN_KERNEL_PREFILL = 3 };
 
 // Cache-policy operands of buffer loads on gfx950: default, or the nontemporal hint (bit 1) for
 // data a launch reads once. Streaming 1 GiB with 16-byte loads measured 6.0 TB/s with the default
@@ -182,6 +182,52 @@ __host__ __device__ inline bool mfma_head_dim(int D, bool bf16) {
 }
 
 hipError_t launch_paged_attention(const AttnArgs& a, int kernel, hipStream_t stream);
+
+// Many query rows per kv head (prefill_attention.hip): rows of a workgroup, and the head dims.
+constexpr int kPrefillRows = 128;
+__host__ __device__ inline bool prefill_head_dim(int D, bool bf16) {
+    return mfma_head_dim(D, true) && (bf16 || D <= 128);
+}
+// Whether a call whose sequences bring `rows` rows per kv head in all goes to it: in bf16 from 192
+// rows a sequence on, or 96 where the batch has 8192 rows over its kv heads. Measured against the
+// kernels that stream K/V per wave (32/8 heads, head dim 128, us): 192 rows 22.9 against 18.5 at
+// one sequence of 1024 tokens, 384 rows 80.8 against 47.5 at 16384; 128 rows of 16 sequences 30.2
+// against 27.0 and 74.6 against 64.7. The f32 one-block kernel at head dim 128 holds out longer
+// (256 rows of four 256-token prompts 27.8 against 29.8; 1024 rows always slower); other f32 head
+// dims have the vector kernel only (32 rows 29.0 against 17.6 us at 1024 tokens).
+inline bool prefill_rows(bool bf16, int D, long long rows, int seqs, int kv_heads) {
+    if (!bf16) return rows >= (D == 128 ? 512LL : 32LL) * seqs;
+    return rows >= 192LL * seqs || (rows >= 96LL * seqs && rows * kv_heads >= 8192);
+}
+// Tokens of a K/V tile: 64, or 32 where a padded row is wider than 256 bytes (two buffers of K
+// and V then take at most 64 KiB of LDS, so that a CU holds two workgroups).
+__host__ __device__ constexpr int prefill_tile_tokens(bool bf16, int D) {
+    return (D + 31) / 32 * 32 * (bf16 ? 2 : 4) <= 256 ? 64 : 32;
+}
+
+// Workgroups of the many-row kernel a CU holds (registers and LDS).
+__host__ __device__ constexpr int prefill_wgs_per_cu(bool bf16, int D) {
+    return bf16 && D <= 64 ? 4 : bf16 && D <= 96 ? 3 : 2;
+}
+
+struct PrefillArgs {
+    AttnArgs a;       // row_groups: kPrefillRows-row groups of the largest q_len; ws_*: partial states,
+                      // [part, kv head, kPrefillRows]
+    int4* list;       // [list_cap][2] {b, q0, q_len, ctx}, {first row, first tile, tiles, part or -1};
+                      // nullptr: every row group of every sequence, the last ones first
+    int4* comb;       // [part_cap][2] {q0, q_len, first row, 0}, {first part, parts, 0, 0}
+    int* head;        // {list entries, split row groups}
+    int list_cap;     // entries the workspace holds
+    int part_cap;     // parts (partial states per kv head) it holds; 0: row groups are not split
+    int splits;       // without a list: parts of a row group at most, part s the tiles from s * chunk on
+    int chunk;
+    int tile_tokens;  // prefill_tile_tokens
+    int slots;        // workgroups the device runs at once
+    int split_cost;   // tiles a workgroup computes in the time that parking and merging one part takes
+};
+
+hipError_t launch_attention_prefill(const PrefillArgs& p, hipStream_t stream);
+
 // The bf16 MFMA kernel at head dims 64, 80, 96 and 256, and at 112, 160, 192 and 224 (a
 // translation unit each).
 hipError_t launch_paged_attention_mfma_hd(const AttnArgs& a, hipStream_t stream);

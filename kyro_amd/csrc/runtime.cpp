@@ -156,14 +156,85 @@ constexpr int kDefaultCUs = 256;  // MI355X; used when no context (device) is gi
 // decomposition, schedule and workspace size. No device call.
 struct AttnSetup {
     kyro::AttnArgs a{};
+    kyro::PrefillArgs pf{};  // ATTN_KERNEL_PREFILL: everything but pf.a
     int kernel = 0;
     bool empty = false;      // nothing to launch (B or total_q is 0)
     size_t plan_slots = 0;   // balanced schedule: partial-state slots sized
     size_t ws_bytes = 0;     // arena bytes the launch takes
 };
 
+// Parts that each of `items` row groups of at most `most` tiles is split into when the host decides
+// alone: the least of an estimate in tile times (one workgroup on a CU: about 1.1 us in bf16, 4 us in
+// f32). Workgroups beyond one a CU share it; a split costs the second launch, and each part its
+// 64 KiB to park and to merge.
+int prefill_splits(long long items, long long most, int num_cus, int wgs_per_cu, bool bf16) {
+    const double fixed = bf16 ? 4.0 : 1.0, each = (bf16 ? 0.025 : 0.007), serial = bf16 ? 0.05 : 0.02;
+    const double share = wgs_per_cu > 2 ? 0.5 : 0.8;
+    double best = 1e30;
+    int best_s = 1;
+    for (int s = 1; s <= 64 && s <= most && (s == 1 || items * s <= (long long)num_cus * wgs_per_cu); ++s) {
+        const long long len = (most + s - 1) / s;
+        const long long per_cu = (items * s + num_cus - 1) / num_cus;
+        double t = (double)len * (1.0 + share * (double)(per_cu - 1));
+        if (s > 1) t += fixed + each * (double)(items * s) + serial * s;
+        if (t < best) {
+            best = t;
+            best_s = s;
+        }
+    }
+    return best_s;
+}
+
+// Work bounds and workspace of a launch of the many-row kernel (prefill_attention.hip). False where
+// a bound passes what one launch carries.
+bool prefill_setup(int num_cus, AttnSetup& s) {
+    kyro::AttnArgs& a = s.a;
+    kyro::PrefillArgs& f = s.pf;
+    f.tile_tokens = kyro::prefill_tile_tokens(a.dtype_bf16, a.D);
+    f.slots = kyro::prefill_wgs_per_cu(a.dtype_bf16, a.D) * num_cus;
+    f.split_cost = a.dtype_bf16 ? 6 : 2;
+    a.rows_per_group = kyro::kPrefillRows;
+    a.row_groups = (a.rows_cap + kyro::kPrefillRows - 1) / kyro::kPrefillRows;
+    const long long all = (long long)a.B * a.row_groups;
+    const long long groups = std::min(all, (long long)a.total_q * a.group / kyro::kPrefillRows + a.B);
+    if (all > INT32_MAX) return false;
+    const long long most = ((long long)a.max_blocks * a.bs + f.tile_tokens - 1) / f.tile_tokens;
+    const size_t acc_row = (size_t)(a.D + 31) / 32 * 32 * sizeof(float);
+    const bool dense = all <= 2 * groups;  // most sequences have about max_q_len rows
+    const bool few = all * a.Hkv <= f.slots;
+    if (dense && (few || most * f.tile_tokens <= (a.dtype_bf16 ? 1024 : 256))) {
+        const int want = few ? prefill_splits(all * a.Hkv, most, num_cus, f.slots / num_cus, a.dtype_bf16) : 1;
+        f.chunk = (int)((most + want - 1) / want);
+        f.chunk = std::max(f.chunk, 1);
+        f.splits = (int)std::max(1LL, (most + f.chunk - 1) / f.chunk);
+        if (all * f.splits * a.Hkv * 256 <= 0xffffffffLL) {
+            f.list_cap = (int)(all * f.splits);
+            f.part_cap = f.splits > 1 ? (int)(all * f.splits) : 0;
+            const size_t rows = (size_t)f.part_cap * a.Hkv * kyro::kPrefillRows;
+            s.ws_bytes = 2 * align_up(rows * sizeof(float), 256) + align_up(rows * acc_row, 256);
+            s.kernel = kyro::ATTN_KERNEL_PREFILL;
+            return true;
+        }
+    }
+    f.splits = f.chunk = 0;
+    // A part is longer than the share ceil(tiles x Hkv / slots), so the row groups that split make
+    // at most 2 x slots / Hkv parts; and each at most ceil(longest / (split_cost + 1)).
+    long long parts = 0;
+    if (most > f.split_cost + 1)
+        parts = std::min(2LL * f.slots / a.Hkv + 2, groups * ((most + f.split_cost) / (f.split_cost + 1)));
+    if ((groups + parts) * a.Hkv * 256 > 0xffffffffLL) return false;
+    f.list_cap = (int)(groups + parts);
+    f.part_cap = (int)parts;
+    const size_t rows = (size_t)parts * a.Hkv * kyro::kPrefillRows;
+    s.ws_bytes = 256 + align_up((size_t)f.list_cap * 2 * sizeof(int4), 256) +
+                 align_up((size_t)f.part_cap * 2 * sizeof(int4), 256) + 2 * align_up(rows * sizeof(float), 256) +
+                 align_up(rows * acc_row, 256);
+    s.kernel = kyro::ATTN_KERNEL_PREFILL;
+    return true;
+}
+
 int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int num_cus, AttnSetup& s,
-                    int chunk_quarters = kyro::kPlanChunkQuarters) {
+                    int chunk_quarters = kyro::kPlanChunkQuarters, bool many_rows = true) {
     if (!p) return fail(KYRO_EINVAL, "paged_attention: params is null");
     if (p->block_size <= 0 || p->num_heads <= 0 || p->head_dim <= 0 || p->num_kv_heads <= 0)
         return fail(KYRO_EINVAL, "paged_attention: block_size/num_heads/head_dim/num_kv_heads must be > 0");
@@ -248,6 +319,16 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     const double scale = p->scale > 0 ? (double)p->scale : 1.0 / std::sqrt((double)p->head_dim);
     a.scale_log2 = (float)(scale * 1.4426950408889634);
     a.units = p->batch_size * p->num_kv_heads;
+    if (many_rows && mfma_blocks && kyro::prefill_head_dim(p->head_dim, p->dtype == KYRO_BF16) &&
+        (p->path == KYRO_ATTN_AUTO || (p->path == KYRO_ATTN_MFMA && mfma_ok)) && p->num_splits <= 0 &&
+        p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (long long)p->max_blocks_per_seq * p->block_size < (1ll << 30) &&
+        kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, (long long)p->total_q * group, p->batch_size, p->num_kv_heads)) {
+        a.ubs = 16;
+        a.sub = a.bs / 16;
+        if (prefill_setup(num_cus, s)) return KYRO_OK;
+        a.ubs = kernel == kyro::ATTN_KERNEL_MFMA ? 16 : p->block_size;
+        a.sub = a.bs / a.ubs;
+    }
     // Row groups: a unit's group * max_q_len query rows are spread over workgroups of 8
     // (vector) or 16 / 32 / 64 / 80 (MFMA) rows that stream the same K/V. The five-tile choice
     // reads the average rows per kv head from total_q (an upper bound when q has padding rows).
@@ -355,6 +436,22 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
 // s.ws_bytes of device memory.
 void attention_workspace(AttnSetup& s, char* base) {
     kyro::AttnArgs& a = s.a;
+    if (s.kernel == kyro::ATTN_KERNEL_PREFILL) {
+        kyro::PrefillArgs& f = s.pf;
+        const size_t rows = (size_t)f.part_cap * a.Hkv * kyro::kPrefillRows;
+        if (!f.splits) {
+            f.head = reinterpret_cast<int*>(base);
+            base += 256;
+            f.list = reinterpret_cast<int4*>(base);
+            base += align_up((size_t)f.list_cap * 2 * sizeof(int4), 256);
+            f.comb = reinterpret_cast<int4*>(base);
+            base += align_up((size_t)f.part_cap * 2 * sizeof(int4), 256);
+        }
+        a.ws_m = reinterpret_cast<float*>(base);
+        a.ws_l = reinterpret_cast<float*>(base + align_up(rows * sizeof(float), 256));
+        a.ws_acc = reinterpret_cast<float*>(base + 2 * align_up(rows * sizeof(float), 256));
+        return;
+    }
     const size_t rows = a.plan ? s.plan_slots * a.hpw * a.plan_rw : (size_t)a.units * a.splits * a.rows_cap;
     const size_t mb_bytes = align_up(rows * sizeof(float), 256);
     a.ws_m = reinterpret_cast<float*>(base);
@@ -636,7 +733,10 @@ int kyro_paged_attention_mq(kyro_ctx ctx, const kyro_paged_attention_params* p, 
     return guarded([&]() -> int {
         if (int rc = check_ctx(ctx)) return rc;
         AttnSetup s;
-        if (int rc = attention_setup(p, q_start_loc != nullptr, ctx->num_cus, s)) return rc;
+        // The many-row kernel copies cache rows to LDS 16 bytes at a time.
+        const bool aligned = ((reinterpret_cast<uintptr_t>(key_cache) | reinterpret_cast<uintptr_t>(value_cache)) & 15) == 0;
+        if (int rc = attention_setup(p, q_start_loc != nullptr, ctx->num_cus, s, kyro::kPlanChunkQuarters, aligned))
+            return rc;
         if (s.empty) return KYRO_OK;
         if (!query || !key_cache || !value_cache || !block_table || !context_lens || !out)
             return fail(KYRO_EINVAL, "paged_attention: null device pointer");
@@ -656,6 +756,11 @@ int kyro_paged_attention_mq(kyro_ctx ctx, const kyro_paged_attention_params* p, 
         }
         if (a.plan) a.sched = ctx->sched;
         a.err = ctx->err;
+        if (s.kernel == kyro::ATTN_KERNEL_PREFILL) {
+            s.pf.a = a;
+            KYRO_HIP(kyro::launch_attention_prefill(s.pf, ctx->stream));
+            return KYRO_OK;
+        }
         KYRO_HIP(kyro::launch_paged_attention(a, s.kernel, ctx->stream));
         return KYRO_OK;
     });
@@ -669,8 +774,14 @@ int kyro_paged_attention_workspace(kyro_ctx ctx, const kyro_paged_attention_para
         // A null context sizes for kDefaultCUs (256) compute units; a device with more needs its
         // context here, since the balanced schedule's persistent grid follows the CU count.
         AttnSetup s;
-        if (int rc = attention_setup(p, has_q_start_loc != 0, ctx ? ctx->num_cus : kDefaultCUs, s)) return rc;
+        const int cus = ctx ? ctx->num_cus : kDefaultCUs;
+        if (int rc = attention_setup(p, has_q_start_loc != 0, cus, s)) return rc;
         *bytes = s.ws_bytes;
+        if (s.kernel == kyro::ATTN_KERNEL_PREFILL) {  // caches that are not 16-byte aligned take another kernel
+            AttnSetup other;
+            if (int rc = attention_setup(p, has_q_start_loc != 0, cus, other, kyro::kPlanChunkQuarters, false)) return rc;
+            *bytes = std::max(*bytes, other.ws_bytes);
+        }
         return KYRO_OK;
     });
 }
@@ -696,7 +807,14 @@ int kyro_paged_attention_describe(kyro_ctx ctx, const kyro_paged_attention_param
         if (s.empty) return put_text("nothing to launch (no sequences or no query rows)", buf, len, needed);
         const kyro::AttnArgs& a = s.a;
         char t[512];
-        if (s.kernel == kyro::ATTN_KERNEL_MFMA) {
+        if (s.kernel == kyro::ATTN_KERNEL_PREFILL) {
+            std::snprintf(t, sizeof t,
+                          "attn_prefill_kernel<%s, head_dim %d> %d rows per workgroup, tiles of %d tokens, row groups %d, "
+                          "parts up to %d, workgroups up to %lld (+ attn_prefill_plan_kernel%s)",
+                          a.dtype_bf16 ? "bf16" : "f32", a.D, kyro::kPrefillRows, s.pf.tile_tokens, a.row_groups,
+                          s.pf.part_cap, (long long)s.pf.list_cap * a.Hkv,
+                          s.pf.part_cap > 0 ? ", attn_prefill_combine_kernel" : "");
+        } else if (s.kernel == kyro::ATTN_KERNEL_MFMA) {
             const int rpg = a.rows_per_group;
             const char* pol = a.stream_kv == kyro::kKvPerUnit ? "per-unit" : a.stream_kv ? "stream" : "cached";
             std::snprintf(t, sizeof t,
