@@ -20,7 +20,7 @@ OBJDIR = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libkyro_verify.so")
 STATIC_LIB = os.path.join(HERE, "libkyro_verify.a")
 SOURCES = ["runtime.cpp", "upload.hip", "blocks_abi.cpp", "block_manager.cpp", "sample_abi.cpp", "ngram_abi.cpp",
-           "paged_attention.hip", "paged_attention_hd.hip", "paged_attention_hd_wide.hip",
+           "paged_attention.hip", "paged_attention_hd.hip", "paged_attention_hd_wide.hip", "paged_attention_hd_f32.hip",
            "prefill_attention.hip", "prefill_attention_wide.hip", "prefill_attention_f32.hip", "spec_verify.hip", "kv_append.hip", "sample.hip", "ngram.hip", "noalloc.hip"]
 ARCH = "gfx950"
 # Per-source flags. paged_attention.hip (the head-dim-128 MFMA kernels, bf16 and f32) takes MFMA

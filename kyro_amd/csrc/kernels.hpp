@@ -181,6 +181,10 @@ __host__ __device__ inline bool mfma_head_dim(int D, bool bf16) {
     return D == 128 || (bf16 && ((D % 32 == 0 && D >= 64 && D <= 256) || D == 80 || D == 112));
 }
 
+// Head dims the f32 MFMA kernel is built for beside 128. Only automatic kernel choice takes it there;
+// a caller that asks for the MFMA kernel or the balanced schedule by name gets it at 128 only.
+inline bool mfma_f32_auto_dim(int D) { return D == 64 || D == 80 || D == 96 || D == 112; }
+
 hipError_t launch_paged_attention(const AttnArgs& a, int kernel, hipStream_t stream);
 
 // Many query rows per kv head (prefill_attention.hip): rows of a workgroup, and the head dims.
@@ -193,18 +197,19 @@ __host__ __device__ inline bool prefill_head_dim(int D, bool bf16) {
 // kernels that stream K/V per wave (32/8 heads, head dim 128, us): 192 rows 22.9 against 18.5 at
 // one sequence of 1024 tokens, 384 rows 80.8 against 47.5 at 16384; 128 rows of 16 sequences 30.2
 // against 27.0 and 74.6 against 64.7. The f32 one-block kernel at head dim 128 holds out longer
-// (256 rows of four 256-token prompts 27.8 against 29.8; 1024 rows always slower); other f32 head
-// dims have the vector kernel only (32 rows 29.0 against 17.6 us at 1024 tokens).
+// (256 rows of four 256-token prompts 27.8 against 29.8; 1024 rows always slower); at
+// the other f32 head dims the two meet between 64 and 128 rows (head dim 64, 16 sequences of 1024
+// tokens: 64 rows 50.9 against 49.7, 128 rows 58.4 against 53.0; of 4096: 143 against 152, 208
+// against 163).
 inline bool prefill_rows(bool bf16, int D, long long rows, int seqs, int kv_heads) {
-    if (!bf16) return rows >= (D == 128 ? 512LL : 32LL) * seqs;
+    if (!bf16) return rows >= (D == 128 ? 512LL : 96LL) * seqs;
     return rows >= 192LL * seqs || (rows >= 96LL * seqs && rows * kv_heads >= 8192);
 }
-// Tokens of a K/V tile: 64, or 32 where a padded row is wider than 256 bytes (two buffers of K
-// and V then take at most 64 KiB of LDS, so that a CU holds two workgroups).
+// Tokens of a K/V tile: 64, or 32 in f32 and where a padded row is wider than 256 bytes (two buffers
+// of K and V then take at most 64 KiB of LDS, so that a CU holds two workgroups).
 __host__ __device__ constexpr int prefill_tile_tokens(bool bf16, int D) {
-    return (D + 31) / 32 * 32 * (bf16 ? 2 : 4) <= 256 ? 64 : 32;
+    return bf16 && D <= 128 ? 64 : 32;
 }
-
 // Workgroups of the many-row kernel a CU holds (registers and LDS).
 __host__ __device__ constexpr int prefill_wgs_per_cu(bool bf16, int D) {
     return bf16 && D <= 64 ? 4 : bf16 && D <= 96 ? 3 : 2;
@@ -232,6 +237,8 @@ hipError_t launch_attention_prefill(const PrefillArgs& p, hipStream_t stream);
 // translation unit each).
 hipError_t launch_paged_attention_mfma_hd(const AttnArgs& a, hipStream_t stream);
 hipError_t launch_paged_attention_mfma_hd_wide(const AttnArgs& a, hipStream_t stream);
+// The f32 one at 64, 80, 96 and 112.
+hipError_t launch_paged_attention_mfma_hd_f32(const AttnArgs& a, hipStream_t stream);
 
 // Per-sequence decision taken after the acceptance scan.
 struct SpecPlan {

@@ -27,7 +27,7 @@
 //    that hold the unit's rows computed), so that such a unit streams its K/V once. The softmax'd S^T fragment is already the P^T operand of the PV
 //    product, and the output column of O^T is the query row, so the per-row rescale stays in the
 //    lane that owns the row's softmax state.
-//  * attn_mfma_f32_kernel (f32, D = 128, block_size 16): the same products on
+//  * attn_mfma_f32_kernel (f32, D = 64, 80, 96, 112 and 128): the same products on
 //    v_mfma_f32_16x16x4_f32, one 16-token block per step;
 //  * attn_vector_kernel (f32 or bf16, D = 64 or 128, any block size): 16 lanes per token row,
 //    4 token rows per wave per step, dot products reduced with DPP inside each 16-lane row.
@@ -1093,24 +1093,38 @@ __device__ __forceinline__ void mfma_item(const AttnArgs& a, Frame<NTW * 16, D> 
 //    the same way for its rows.
 //  * O^T += V^T P^T over tokens 4 g + q at step q (q = 0..3): the softmax'd S^T fragment of lane
 //    (row r, g) holds tokens 4 g + e, so element q is already the B operand of step q (no
-//    shuffle). Lane (r, g) loads V[token 4 g + q][64 h + 4 r .. + 3] (h = 0, 1): component e_t
-//    is the A operand of the d-tile holding dims 64 h + 4 i + e_t, and the accumulator of that
-//    tile gives lane (r, g) dims 64 h + 16 g + 4 e' + e_t of row r.
+//    shuffle). Lane (r, g) loads V[token 4 g + q] by column groups (F32Cols: at head dim 128
+//    dims 64 h + 4 r .. + 3 for h = 0, 1): component j is the A operand of the d-tile that holds
+//    every 4th (2nd, single) column of the group from j on.
 // 32 + 32 MFMAs per block and 16-row tile: at 32 cycles each, about 60% of a block's streaming
 // time for two tiles (GQA 32/8 with 8 draft rows), so the loads still set the pace.
 
 __device__ float kZeroSlabF32[kMfmaBS * kMfmaD];
 
-struct KVBlockF32 {
-    float4 k[8];  // [s]: token r, dims 16 s + 4 g .. + 3
-    float4 v[8];  // [2 q + h]: token 4 g + q, dims 64 h + 4 r .. + 3
+// Column groups of V and O: as many 64-column groups as fit, then one of 32 and one of 16 (head dims
+// are multiples of 16). Lane r holds 4, 2 or 1 consecutive columns of a group, so that a load
+// instruction covers whole runs of a token row; d-tile dt is column j of group base.
+template <int D>
+struct F32Cols {
+    static constexpr int k64 = D / 64, k32 = D % 64 / 32, k16 = D % 32 / 16;
+    static constexpr int T = D / 16;  // d-tiles
+    static constexpr int base(int dt) { return dt < 4 * k64 ? dt / 4 * 64 : dt < 4 * k64 + 2 * k32 ? 64 * k64 : D - 16; }
+    static constexpr int width(int dt) { return dt < 4 * k64 ? 4 : dt < 4 * k64 + 2 * k32 ? 2 : 1; }
+    static constexpr int j(int dt) { return dt < 4 * k64 ? dt % 4 : dt < 4 * k64 + 2 * k32 ? (dt - 4 * k64) % 2 : 0; }
 };
 
-template <int POL>
-__device__ __forceinline__ void load_block_f32(KVBlockF32& kv, const float* __restrict__ kp,
+template <int D>
+struct KVBlockF32 {
+    float4 k[D / 16];    // [s]: token r, dims 16 s + 4 g .. + 3
+    float v[4][D / 16];  // [q][dt]: token 4 g + q, column base(dt) + width(dt) r + j(dt)
+};
+
+template <int POL, int D>
+__device__ __forceinline__ void load_block_f32(KVBlockF32<D>& kv, const float* __restrict__ kp,
                                                const float* __restrict__ vp, int blk, size_t slot_stride,
                                                size_t kv_off, int r, int g) {
-    constexpr int kSlabBytes = kMfmaBS * kMfmaD * 4;
+    using Cols = F32Cols<D>;
+    constexpr int kSlabBytes = kMfmaBS * D * 4;
     const size_t base = (size_t)(blk >= 0 ? blk : 0) * slot_stride + kv_off;
     const float* kslab = blk >= 0 ? kp + base : kZeroSlabF32;
     const float* vslab = blk >= 0 ? vp + base : kZeroSlabF32;
@@ -1118,17 +1132,32 @@ __device__ __forceinline__ void load_block_f32(KVBlockF32& kv, const float* __re
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kslab), (short)0, kSlabBytes, kRawBufferWord3);
     const __amdgpu_buffer_rsrc_t vr =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vslab), (short)0, kSlabBytes, kRawBufferWord3);
-    const int koff = (r * kMfmaD + 4 * g) * 4;       // + 64 s
-    const int voff = (4 * g * kMfmaD + 4 * r) * 4;   // + (q * 128 + 64 h) * 4
+    const int koff = (r * D + 4 * g) * 4;  // + 64 s
+    const int vrow = 4 * g * D * 4;        // + q D * 4
 #pragma unroll
-    for (int s = 0; s < 8; ++s)
+    for (int s = 0; s < D / 16; ++s)
         kv.k[s] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(kr, koff, 64 * s, POL));
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 4; ++q) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-            kv.v[2 * q + h] =
-                __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(vr, voff, (q * kMfmaD + 64 * h) * 4, POL));
+        for (int h = 0; h < Cols::k64; ++h) {
+            const float4 x = __builtin_bit_cast(
+                float4, __builtin_amdgcn_raw_buffer_load_b128(vr, vrow + 16 * r, (q * D + 64 * h) * 4, POL));
+            kv.v[q][4 * h] = x.x;
+            kv.v[q][4 * h + 1] = x.y;
+            kv.v[q][4 * h + 2] = x.z;
+            kv.v[q][4 * h + 3] = x.w;
+        }
+        if constexpr (Cols::k32 > 0) {
+            const float2 x = __builtin_bit_cast(
+                float2, __builtin_amdgcn_raw_buffer_load_b64(vr, vrow + 8 * r, (q * D + 64 * Cols::k64) * 4, POL));
+            kv.v[q][4 * Cols::k64] = x.x;
+            kv.v[q][4 * Cols::k64 + 1] = x.y;
+        }
+        if constexpr (Cols::k16 > 0)
+            kv.v[q][Cols::T - 1] =
+                __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(vr, vrow + 4 * r, (q * D + D - 16) * 4, POL));
+    }
 }
 
 __device__ __forceinline__ float f4_get(const float4& v, int i) {
@@ -1136,11 +1165,17 @@ __device__ __forceinline__ float f4_get(const float4& v, int i) {
 }
 
 // One work item of the f32 kernel; the arguments are those of mfma_item.
-template <int NTW, int HP, int POL>
-__device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16, kMfmaD> (&frame)[HP], int* s_blk,
+template <int NTW, int HP, int POL, int D>
+__device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16, D> (&frame)[HP], int* s_blk,
                                               const SeqInfo& si, int ug, int rg, int blk_begin, int blk_end,
                                               int nsplit, size_t pb0, size_t pbstep) {
-    constexpr int D = kMfmaD;
+    using Cols = F32Cols<D>;
+    constexpr int T = Cols::T;
+    // At the other head dims the kernel stands in for the vector kernel, whose sums are trees: four
+    // chains per score and one per block and output keep its error against 64 bits (16 sequences of
+    // 300-3000 tokens, head dim 64: 2.13e-7 in the vector kernel, 1.91e-7 here). That batch went
+    // from 143 to 31.6 us: the vector kernel spends a shuffle tree per row and token.
+    constexpr bool kShort = D != kMfmaD;
     constexpr int RW = NTW * 16;
     constexpr int WPH = kWaves / HP;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1163,7 +1198,7 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
 
     {
         // Q^T operands: lane (r, g) holds row row0 + 16 nt + r, dims 16 s + 4 g .. + 3.
-        float4 qB[NTW][8];
+        float4 qB[NTW][T];
         int vis[NTW];
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt) {
@@ -1172,36 +1207,41 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
                 const int j = n / a.group;
                 const size_t qrow = out_row(a, si, n);
 #pragma unroll
-                for (int s = 0; s < 8; ++s) qB[nt][s] = *reinterpret_cast<const float4*>(qp + qrow * D + 16 * s + 4 * g);
+                for (int s = 0; s < T; ++s) qB[nt][s] = *reinterpret_cast<const float4*>(qp + qrow * D + 16 * s + 4 * g);
                 vis[nt] = a.causal ? si.ctx - si.q_len + j + 1 : si.ctx;
             } else {
 #pragma unroll
-                for (int s = 0; s < 8; ++s) qB[nt][s] = make_float4(0.f, 0.f, 0.f, 0.f);
+                for (int s = 0; s < T; ++s) qB[nt][s] = make_float4(0.f, 0.f, 0.f, 0.f);
                 vis[nt] = si.ctx;
             }
         }
 
         float m[NTW], lsum[NTW];
-        f32x4 O[8][NTW];  // [2 h + ... ] d-tile dt = 4 h + e_t
+        f32x4 O[T][NTW];  // by d-tile
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt) {
             m[nt] = kNegInf;
             lsum[nt] = 0.f;
 #pragma unroll
-            for (int dt = 0; dt < 8; ++dt) O[dt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int dt = 0; dt < T; ++dt) O[dt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 
-        auto compute = [&](KVBlockF32& kv, int pb, int blk) {
+        auto compute = [&](KVBlockF32<D>& kv, int pb, int blk) {
             f32x4 S[NTW];
 #pragma unroll
             for (int nt = 0; nt < NTW; ++nt) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                constexpr int NC = kShort ? 4 : 1;
+                f32x4 acc[NC];
 #pragma unroll
-                for (int s = 0; s < 8; ++s)
+                for (int x = 0; x < NC; ++x) acc[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < T; ++s)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(f4_get(kv.k[s], e), f4_get(qB[nt][s], e), acc, 0, 0, 0);
-                S[nt] = acc;
+                        acc[e % NC] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4_get(kv.k[s], e), f4_get(qB[nt][s], e),
+                                                                           acc[e % NC], 0, 0, 0);
+                if constexpr (kShort) S[nt] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+                else S[nt] = acc[0];
             }
             const bool full = blk >= 0 && (pb + 1) * kMfmaBS <= full_vis;
             if (!full) {
@@ -1209,8 +1249,8 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     if (pb * kMfmaBS + 4 * g + q >= si.ctx) {
-                        kv.v[2 * q] = make_float4(0.f, 0.f, 0.f, 0.f);
-                        kv.v[2 * q + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                        for (int dt = 0; dt < T; ++dt) kv.v[q][dt] = 0.f;
                     }
             }
             float pv[NTW][4];
@@ -1240,19 +1280,30 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
                 lsum[nt] = lsum[nt] * alpha + ps;
                 if (__any(m_new > m[nt] && m[nt] != kNegInf)) {
 #pragma unroll
-                    for (int dt = 0; dt < 8; ++dt) O[dt][nt] *= alpha;
+                    for (int dt = 0; dt < T; ++dt) O[dt][nt] *= alpha;
                 }
                 m[nt] = m_new;
             }
+            if constexpr (kShort) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+                for (int dt = 0; dt < T; ++dt)
 #pragma unroll
-                for (int dt = 0; dt < 8; ++dt) {
-                    const float av = f4_get(kv.v[2 * q + (dt >> 2)], dt & 3);
+                    for (int nt = 0; nt < NTW; ++nt) {
+                        f32x4 add = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int nt = 0; nt < NTW; ++nt)
-                        O[dt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, pv[nt][q], O[dt][nt], 0, 0, 0);
-                }
+                        for (int q = 0; q < 4; ++q)
+                            add = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.v[q][dt], pv[nt][q], add, 0, 0, 0);
+                        O[dt][nt] += add;
+                    }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int dt = 0; dt < T; ++dt)
+#pragma unroll
+                        for (int nt = 0; nt < NTW; ++nt)
+                            O[dt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.v[q][dt], pv[nt][q], O[dt][nt], 0, 0, 0);
+            }
         };
 
         // Each wave streams blocks wp, wp + WPH, ... of the split; the next block's loads are issued
@@ -1281,18 +1332,18 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
                 const int x = block_id(min(j + 1, kSlots * 64 - 1));
                 return j + 1 < nblk ? x : -1;
             };
-            KVBlockF32 bufA, bufB;
+            KVBlockF32<D> bufA, bufB;
             if (nblk > 0) {
                 int j = 0;
                 int ia = block_id(0), ib;
-                load_block_f32<POL>(bufA, kp, vp, ia, slot_stride, kv_off, r, g);
+                load_block_f32<POL, D>(bufA, kp, vp, ia, slot_stride, kv_off, r, g);
                 while (true) {
                     ib = next_id(j);
-                    load_block_f32<POL>(bufB, kp, vp, ib, slot_stride, kv_off, r, g);
+                    load_block_f32<POL, D>(bufB, kp, vp, ib, slot_stride, kv_off, r, g);
                     compute(bufA, b0 + j * WPH, ia);
                     if (++j >= nblk) break;
                     ia = next_id(j);
-                    load_block_f32<POL>(bufA, kp, vp, ia, slot_stride, kv_off, r, g);
+                    load_block_f32<POL, D>(bufA, kp, vp, ia, slot_stride, kv_off, r, g);
                     compute(bufB, b0 + j * WPH, ib);
                     if (++j >= nblk) break;
                 }
@@ -1324,22 +1375,20 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
                 if (wp == 0) fr.mx[n] = M;
             }
         }
-        // Lane (r, g) holds dims 64 h + 16 g + 4 e' + e_t of row 16 nt + r in O[4 h + e_t][nt][e'].
+        // Lane (r, g) holds column base(dt) + width(dt) (4 g + e) + j(dt) of row 16 nt + r in O[dt][nt][e].
         for (int w = 0; w < WPH; ++w) {
             if (wp == w) {
 #pragma unroll
                 for (int nt = 0; nt < NTW; ++nt) {
-                    float* dst = &fr.acc[(nt * 16 + r) * Frame<RW, D>::kStride + 16 * g];
+                    float* dst = &fr.acc[(nt * 16 + r) * Frame<RW, D>::kStride];
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
+                    for (int dt = 0; dt < T; ++dt)
 #pragma unroll
-                        for (int e2 = 0; e2 < 4; ++e2)
-#pragma unroll
-                            for (int et = 0; et < 4; ++et) {
-                                const float v = O[4 * h + et][nt][e2] * f[nt];
-                                float* p = dst + 64 * h + 4 * e2 + et;
-                                *p = (w == 0) ? v : *p + v;
-                            }
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = O[dt][nt][e] * f[nt];
+                            float* p = dst + Cols::base(dt) + Cols::width(dt) * (4 * g + e) + Cols::j(dt);
+                            *p = (w == 0) ? v : *p + v;
+                        }
                 }
             }
             __syncthreads();
@@ -1481,13 +1530,13 @@ __global__ __launch_bounds__(kThreads) void attn_mfma_kernel(AttnArgs a) {
 }
 
 // f32 caches.
-template <int NTW, int HP, int POL, bool PLAN>
+template <int NTW, int HP, int POL, bool PLAN, int D = kMfmaD>
 __global__ __launch_bounds__(kThreads) void attn_mfma_f32_kernel(AttnArgs a) {
-    __shared__ Frame<NTW * 16, kMfmaD> frame[HP];
+    __shared__ Frame<NTW * 16, D> frame[HP];
     __shared__ int s_blk[kMaxChunkBlocks];
     mfma_schedule<NTW, HP, PLAN>(a, [&](const SeqInfo& si, int ug, int rg, int bb, int be, int ns, size_t pb0,
                                         size_t pbs) {
-        mfma_item_f32<NTW, HP, POL>(a, frame, s_blk, si, ug, rg, bb, be, ns, pb0, pbs);
+        mfma_item_f32<NTW, HP, POL, D>(a, frame, s_blk, si, ug, rg, bb, be, ns, pb0, pbs);
     });
 }
 
@@ -1727,14 +1776,19 @@ __global__ __launch_bounds__(kThreads) void attn_vector_kernel(AttnArgs a) {
 // register file), one or two kv heads per workgroup, streaming or cached K/V loads, grid or
 // balanced schedule. D is the operand layout, DR the head dim (80 runs in the layout of 96, 112
 // in that of 128).
-template <int D, int DR = D>
+template <int D, int DR = D, bool BF16 = true>
 hipError_t launch_mfma_hd(const AttnArgs& a, const dim3 grid, hipStream_t stream) {
     const dim3 block(kThreads);
     const int rpg = a.rows_per_group;
 #define KYRO_HD_LAUNCH(NT, POL, PLAN)                                                           \
     {                                                                                           \
-        if (a.hpw == 2) attn_mfma_kernel<NT, 2, POL, PLAN, D, DR><<<grid, block, 0, stream>>>(a); \
-        else attn_mfma_kernel<NT, 1, POL, PLAN, D, DR><<<grid, block, 0, stream>>>(a);          \
+        if constexpr (BF16) {                                                                   \
+            if (a.hpw == 2) attn_mfma_kernel<NT, 2, POL, PLAN, D, DR><<<grid, block, 0, stream>>>(a); \
+            else attn_mfma_kernel<NT, 1, POL, PLAN, D, DR><<<grid, block, 0, stream>>>(a);      \
+        } else {                                                                                \
+            if (a.hpw == 2) attn_mfma_f32_kernel<NT, 2, POL, PLAN, D><<<grid, block, 0, stream>>>(a); \
+            else attn_mfma_f32_kernel<NT, 1, POL, PLAN, D><<<grid, block, 0, stream>>>(a);      \
+        }                                                                                       \
     }
 #define KYRO_HD_POL(NT, PLAN)                                                               \
     {                                                                                       \
@@ -1782,6 +1836,18 @@ hipError_t launch_paged_attention_mfma_hd(const AttnArgs& a, hipStream_t stream)
         default: return hipErrorInvalidValue;
     }
 }
+#elif KYRO_ATTN_HD_UNIT == 3
+hipError_t launch_paged_attention_mfma_hd_f32(const AttnArgs& a, hipStream_t stream) {
+    const dim3 grid((unsigned)(a.plan ? a.plan_grid : a.ugroups_padded * a.splits * a.row_groups));
+    if (grid.x == 0) return hipSuccess;
+    switch (a.D) {
+        case 64: return launch_mfma_hd<64, 64, false>(a, grid, stream);
+        case 80: return launch_mfma_hd<80, 80, false>(a, grid, stream);
+        case 96: return launch_mfma_hd<96, 96, false>(a, grid, stream);
+        case 112: return launch_mfma_hd<112, 112, false>(a, grid, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
 #else
 hipError_t launch_paged_attention_mfma_hd_wide(const AttnArgs& a, hipStream_t stream) {
     const dim3 grid((unsigned)(a.plan ? a.plan_grid : a.ugroups_padded * a.splits * a.row_groups));
@@ -1804,6 +1870,7 @@ hipError_t launch_paged_attention(const AttnArgs& a, int path, hipStream_t strea
     const dim3 block(kThreads);
     const dim3 grid((unsigned)(a.plan ? a.plan_grid : a.ugroups_padded * a.splits * a.row_groups));
     if (grid.x == 0) return hipSuccess;
+    if (path == ATTN_KERNEL_MFMA && a.D != kMfmaD && !a.dtype_bf16) return launch_paged_attention_mfma_hd_f32(a, stream);
     if (path == ATTN_KERNEL_MFMA && a.D != kMfmaD)
         return (a.D == 112 || a.D == 160 || a.D == 192 || a.D == 224) ? launch_paged_attention_mfma_hd_wide(a, stream)
                                                                        : launch_paged_attention_mfma_hd(a, stream);

@@ -11,9 +11,7 @@
 //     before is computed; one barrier per tile. S^T = K Q^T puts a query row in one lane pair
 //     (l, l + 32), so the softmax needs one cross-lane swap, and its S^T fragment is already the
 //     P^T operand of O^T += V^T P^T. bf16 V is read in operand layout by the transposing LDS
-//     loads (ds_read_b64_tr_b16). The running maximum may lag the true one by up to 2^8 (a
-//     factor that cancels in the final division): the accumulator is rescaled only when a row's
-//     maximum rose by more, which after the first tiles almost never happens.
+//     loads (ds_read_b64_tr_b16).
 //   * attn_prefill_plan_kernel: one workgroup lists the work: for each (sequence, row group)
 //     its tiles up to the last visible token, in parts of at most the per-workgroup share of the
 //     total, ordered longest first, so that the dispatcher's in-order hand-out keeps all CUs busy
@@ -72,7 +70,7 @@ struct PfCfg {
     static constexpr int TK = prefill_tile_tokens(BF16, DR);
     static constexpr int NS = TK / kPfBS;            // slabs of a tile
     static constexpr int TT = TK / 32;               // 32-token tiles of S^T
-    static constexpr int SC = DR > 96 ? 2 : 4;  // f32: accumulators per score (registers)
+    static constexpr int SC = DR > 96 ? 2 : 8;       // f32: accumulators per score (what registers allow)
     // K rows: chunk c of token t sits in slot c ^ swk(t) of its column group, so that the 16
     // tokens of an operand read (same c) spread over all banks.
     __device__ static constexpr int swk(int t) { return t * CW / 16; }
@@ -136,19 +134,16 @@ template <class C>
 struct PfState {
     f32x16 o[C::DT];  // O^T: column = the lane's row, rows 32 dt + 8 (i / 4) + 4 h + i % 4
     float m;          // reference the weights are relative to (log2 units, scaled)
-    float top;        // bf16: running maximum
+    float top;        // running maximum
     float l;          // this lane's share of the row sum
 };
-// f32: the reference follows the running maximum only when that rose by more than kLag (a factor of
-// up to 2^kLag in every term, which the final division cancels), which after the first tiles it
-// almost never does. bf16: the reference is the tile's own maximum, so that the largest weight of
-// every tile is 1 and rounds to bf16 exactly. That costs a rescale of O^T per tile (four 2048-token
-// prompts, head dim 128: 169.6 -> 178 us) and lowers the error against 64 bits from 2.09e-3 with the
-// lagging reference and 2.03e-3 with one running maximum to 1.98e-3, where the kernels that stream
-// K/V per wave have 1.97e-3 (contexts of 700-8000 tokens: 2.33e-3, 2.23e-3, 2.09e-3, 2.19e-3). It
-// stays within 2^kDrop of the running maximum, so that O^T
-// and l cannot overflow after a much larger score.
-constexpr float kLag = 8.f;
+// The weights of a tile are relative to the tile's own maximum, so that the largest is 1, which bf16
+// holds exactly. That costs a rescale of O^T per tile (four 2048-token prompts, head dim 128:
+// 169.6 us with a reference that may lag the maximum by 2^8 and so hardly ever moves, 178 so) and
+// lowers the error against 64 bits from 2.09e-3 with the lagging reference and 2.03e-3 with one
+// running maximum to 1.98e-3, where the kernels that stream K/V per wave have 1.97e-3 (contexts of
+// 700-8000 tokens: 2.33e-3, 2.23e-3, 2.09e-3, 2.19e-3). The reference stays within 2^kDrop of the
+// running maximum, so that O^T and l cannot overflow after a much larger score.
 constexpr float kDrop = 30.f;
 
 template <bool BF16, int DR>
@@ -317,31 +312,27 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
             }
             __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
         } else {
-            // Several short chains per score instead of one of DR / 2 sequential additions, as the
-            // vector kernel's tree sums have (f32, head dim 64, error against 64 bits: 3.5e-7 with one
-            // chain here and per output below, 1.7e-7 so, 1.6e-7 in the vector kernel).
-            f32x16 part[C::TT][C::SC];
+            // Several short chains per score instead of one of DR / 2 sequential additions, in step with
+            // the vector kernel's tree sums (head dim 64, error against 64 bits: 3.5e-7 with one chain
+            // here and per output below, 1.6e-7 so and in the vector kernel).
+            static_assert(BF16 || C::TT == 1, "one 32-token tile of scores at a time");
+            f32x16 part[C::SC];
 #pragma unroll
-            for (int tt = 0; tt < C::TT; ++tt)
+            for (int y = 0; y < C::SC; ++y)
 #pragma unroll
-                for (int y = 0; y < C::SC; ++y)
+                for (int x = 0; x < 16; ++x) part[y][x] = 0.f;
 #pragma unroll
-                    for (int x = 0; x < 16; ++x) part[tt][y][x] = 0.f;
+            for (int s = 0; s < C::KS; ++s) {
+                const f32x4 kf = __builtin_bit_cast(f32x4, k_operand(s, 0)), qf = __builtin_bit_cast(f32x4, q[s]);
 #pragma unroll
-            for (int s = 0; s < C::KS; ++s)
-#pragma unroll
-                for (int tt = 0; tt < C::TT; ++tt) {
-                    const f32x4 kf = __builtin_bit_cast(f32x4, k_operand(s, tt)), qf = __builtin_bit_cast(f32x4, q[s]);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        part[tt][e % C::SC] =
-                            __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[e], part[tt][e % C::SC], 0, 0, 0);
+                for (int e = 0; e < 4; ++e) {
+                    f32x16& to = part[(4 * s + e) % C::SC];
+                    to = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[e], to, 0, 0, 0);
                 }
-#pragma unroll
-            for (int tt = 0; tt < C::TT; ++tt) {
-                if constexpr (C::SC == 4) S[tt] = (part[tt][0] + part[tt][1]) + (part[tt][2] + part[tt][3]);
-                else S[tt] = part[tt][0] + part[tt][1];
             }
+            if constexpr (C::SC == 8)
+                S[0] = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+            else S[0] = part[0] + part[1];
         }
         if (t0 + C::TK > wave_lo || tbad) {
 #pragma unroll
@@ -363,23 +354,15 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
             mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
         }
         mx *= c;
-        if constexpr (BF16) {
-            st.top = fmaxf(st.top, mx);
-            const float m_new = fmaxf(mx, st.top - kDrop);
-            // -inf - -inf (nothing visible yet) would be NaN; O^T and l are 0 then.
-            const float alpha = st.m == kNegInf ? 0.f : fast_exp2(st.m - m_new);
+        st.top = fmaxf(st.top, mx);
+        float m_new = fmaxf(mx, st.top - kDrop);
+        if constexpr (!BF16) m_new = ceilf(m_new);  // the rescale is then by a power of two: exact
+        // -inf - -inf (nothing visible yet) would be NaN; O^T and l are 0 then.
+        const float alpha = st.m == kNegInf ? 0.f : fast_exp2(st.m - m_new);
 #pragma unroll
-            for (int dt = 0; dt < C::DT; ++dt) st.o[dt] *= alpha;
-            st.l *= alpha;
-            st.m = m_new;
-        } else if (__any(mx > st.m + kLag)) {
-            const float m_new = fmaxf(st.m, mx);
-            const float alpha = fast_exp2(st.m - (m_new == kNegInf ? 0.f : m_new));
-#pragma unroll
-            for (int dt = 0; dt < C::DT; ++dt) st.o[dt] *= alpha;
-            st.l *= alpha;
-            st.m = m_new;
-        }
+        for (int dt = 0; dt < C::DT; ++dt) st.o[dt] *= alpha;
+        st.l *= alpha;
+        st.m = m_new;
         const float mref = st.m == kNegInf ? 0.f : st.m;
         float ps = 0.f;
 #pragma unroll
@@ -420,33 +403,26 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
         } else {
             // A tile's products are summed on their own and then added: the chain of additions into
             // O^T is one per tile instead of one per two tokens.
-            constexpr int W = C::TT == 2 || C::DT % 2 ? 1 : 2;  // column tiles side by side
+            constexpr int W = C::DT % 2 ? 1 : 2;  // column tiles side by side
 #pragma unroll
             for (int d0 = 0; d0 < C::DT; d0 += W) {
-                f32x16 add[C::TT][W];
+                f32x16 add[W];
 #pragma unroll
-                for (int tt = 0; tt < C::TT; ++tt)
+                for (int w = 0; w < W; ++w)
 #pragma unroll
-                    for (int w = 0; w < W; ++w)
-#pragma unroll
-                        for (int x = 0; x < 16; ++x) add[tt][w][x] = 0.f;
+                    for (int x = 0; x < 16; ++x) add[w][x] = 0.f;
 #pragma unroll
                 for (int x = 0; x < 16; ++x)
 #pragma unroll
-                    for (int tt = 0; tt < C::TT; ++tt)
+                    for (int w = 0; w < W; ++w) {
+                        const int dt = d0 + w;
+                        const float vv = *reinterpret_cast<const float*>(
+                            vb + vaddr32 + (x / 8) * (C::SLAB * 16) + (8 * dt / C::CW) * kGroupBytes +
+                            (8 * ((x / 4) % 2) + x % 4) * (C::CW * 16) + (8 * dt % C::CW) * 16);
+                        add[w] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, S[0][x], add[w], 0, 0, 0);
+                    }
 #pragma unroll
-                        for (int w = 0; w < W; ++w) {
-                            const int dt = d0 + w;
-                            const float vv = *reinterpret_cast<const float*>(
-                                vb + vaddr32 + (2 * tt + x / 8) * (C::SLAB * 16) + (8 * dt / C::CW) * kGroupBytes +
-                                (8 * ((x / 4) % 2) + x % 4) * (C::CW * 16) + (8 * dt % C::CW) * 16);
-                            add[tt][w] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, S[tt][x], add[tt][w], 0, 0, 0);
-                        }
-#pragma unroll
-                for (int w = 0; w < W; ++w) {
-                    if constexpr (C::TT == 2) st.o[d0 + w] += add[0][w] + add[1][w];
-                    else st.o[d0 + w] += add[0][w];
-                }
+                for (int w = 0; w < W; ++w) st.o[d0 + w] += add[w];
             }
         }
     };

@@ -201,7 +201,7 @@ bool prefill_setup(int num_cus, AttnSetup& s) {
     const long long most = ((long long)a.max_blocks * a.bs + f.tile_tokens - 1) / f.tile_tokens;
     const size_t acc_row = (size_t)(a.D + 31) / 32 * 32 * sizeof(float);
     const bool dense = all <= 2 * groups;  // most sequences have about max_q_len rows
-    const bool few = all * a.Hkv <= f.slots;
+    const bool few = all * a.Hkv * 2 <= f.slots;
     if (dense && (few || most * f.tile_tokens <= (a.dtype_bf16 ? 1024 : 256))) {
         const int want = few ? prefill_splits(all * a.Hkv, most, num_cus, f.slots / num_cus, a.dtype_bf16) : 1;
         f.chunk = (int)((most + want - 1) / want);
@@ -292,7 +292,9 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
         // MFMA wherever it applies, one query row per kv head included: the kernel is
         // memory-bound, so padding rows to a 16-row tile costs nothing measurable (MHA decode,
         // 1 row per kv head: 67 us against the vector kernel's 207 us).
-        kernel = mfma_ok ? kyro::ATTN_KERNEL_MFMA : kyro::ATTN_KERNEL_VECTOR;
+        const bool f32_auto = mfma_blocks && p->dtype == KYRO_F32 && kyro::mfma_f32_auto_dim(p->head_dim) &&
+                              p->schedule != KYRO_ATTN_SCHEDULE_BALANCED;
+        kernel = mfma_ok || f32_auto ? kyro::ATTN_KERNEL_MFMA : kyro::ATTN_KERNEL_VECTOR;
     }
     if (p->schedule == KYRO_ATTN_SCHEDULE_BALANCED && kernel != kyro::ATTN_KERNEL_MFMA)
         return fail(KYRO_EUNSUPPORTED, "paged_attention: the balanced schedule runs on the MFMA kernel "
