@@ -393,6 +393,33 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     int chunk = (mb + splits - 1) / splits;
     chunk = std::min((chunk + 1) / 2 * 2, max_chunk);
     splits = (mb + chunk - 1) / chunk;
+    // Where the whole batch's chunks of 8, 16 or 32 slots fit the chip at once, the grid takes them:
+    // no workgroup has more to do than one chunk, whatever the lengths, so there is nothing for the
+    // balanced schedule to even out and its plan (about 5 us in every workgroup) is saved. The
+    // splits stay few enough that the combine pass does not cost more: 32, or 16 with several row
+    // groups or wide heads. One sequence of 1000 tokens, 32/8 heads, bf16: 16.3 -> 14.5 us a call
+    // (the host's time for two launches; 16 -> 9 us of kernels), f32 26.0 -> 14.8, head dim 256
+    // 31.8 -> 19.4; 12000 tokens, 8/8 heads: 21.5 -> 15.7 with 24 splits, but 25.8 against 22.5
+    // with 94 at 32/8 heads. Short bf16 contexts that took one launch before (up to 496 tokens) keep
+    // it: 300 tokens 11.9 us, 14.6 in chunks (f32 20.1 and 14.8).
+    bool short_chunks = false;
+    if (kernel == kyro::ATTN_KERNEL_MFMA && p->num_splits == 0 && p->schedule == KYRO_ATTN_SCHEDULE_AUTO &&
+        (splits > 1 || p->dtype == KYRO_F32 || p->head_dim > 128)) {
+        const long long groups = (long long)a.ugroups * a.row_groups;
+        const bool narrow = a.row_groups == 1 && p->head_dim <= 128;
+        for (int c : {8, 16, 32}) {
+            const int n = (mb + c - 1) / c;
+            if (n < 2 || n > (narrow ? 32 : 16) || groups * n > num_cus) continue;
+            // 32 slots only where the balanced schedule's own chunk (5/4 of a CU's share) would be
+            // about as long: at few groups its shorter ones win (12000 tokens, 32/8 heads, f32: 33.0
+            // against 40.0 us).
+            if (c == 32 && (!narrow || groups * mb * 5 < 96LL * num_cus)) continue;
+            chunk = c;
+            splits = n;
+            short_chunks = true;
+            break;
+        }
+    }
     a.splits = splits;
     a.chunk_blocks = chunk;
     // The balanced schedule: asked for, or where the grid's splits (from the table width
@@ -401,7 +428,7 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     // long after the rest of the chip is idle.
     a.plan = kernel == kyro::ATTN_KERNEL_MFMA && p->num_splits == 0 && p->batch_size <= kyro::kPlanMaxSeqs &&
              (p->schedule == KYRO_ATTN_SCHEDULE_BALANCED ||
-              (p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (splits > 1 || mb > 256)));
+              (p->schedule == KYRO_ATTN_SCHEDULE_AUTO && !short_chunks && (splits > 1 || mb > 256)));
     if (a.plan) {
         // One persistent workgroup per CU, in whole rounds of the 8 XCD lanes the plan deals
         // to (a partitioned device with fewer CUs still gets every lane covered).
