@@ -9,6 +9,8 @@ import ctypes
 import os
 import threading
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # KYRO_VERIFY_LIB names another build of the same library (the tests' host sanitizer run).
 LIB_PATH = os.environ.get("KYRO_VERIFY_LIB") or os.path.join(_HERE, "libkyro_verify.so")
@@ -210,6 +212,12 @@ class Context:
             self.close()
         except Exception:
             pass
+
+
+def current_stream(index: int) -> int:
+    """The hipStream_t handle of torch's current stream on a device, without the Stream object that
+    torch.cuda.current_stream makes (2.0 us a call, 0.2 so)."""
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 _contexts: dict = {}

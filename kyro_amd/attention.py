@@ -87,13 +87,28 @@ class PagedAttention:
         dev = query.device
         if dev.type != "cuda":
             raise ValueError("PagedAttention.forward runs on a GPU device; got " + str(dev))
-        _require(query, "query", dtype=(torch.float32, torch.bfloat16), ndim=3)
-        _require(key_cache, "key_cache", dtype=query.dtype, ndim=4, device=dev)
-        _require(value_cache, "value_cache", dtype=query.dtype, ndim=4, device=dev)
-        _require(block_table, "block_table", dtype=torch.int64, ndim=2, device=dev)
-        _require(context_lens, "context_lens", dtype=torch.int64, ndim=1, device=dev)
-        if key_cache.shape != value_cache.shape:
-            raise ValueError("key_cache and value_cache shapes differ")
+        # One expression for a call whose tensors are as they should be; _require names what is not.
+        dtype = getattr(query, "dtype", None)
+        try:
+            plain = (dtype in _DTYPES and query.dim() == 3 and query.is_contiguous()
+                     and key_cache.dtype == dtype and value_cache.dtype == dtype
+                     and key_cache.dim() == 4 and key_cache.shape == value_cache.shape
+                     and key_cache.is_contiguous() and value_cache.is_contiguous()
+                     and block_table.dtype == torch.int64 and context_lens.dtype == torch.int64
+                     and block_table.dim() == 2 and context_lens.dim() == 1
+                     and block_table.is_contiguous() and context_lens.is_contiguous()
+                     and key_cache.device == dev and value_cache.device == dev
+                     and block_table.device == dev and context_lens.device == dev)
+        except AttributeError:  # not a tensor
+            plain = False
+        if not plain:
+            _require(query, "query", dtype=(torch.float32, torch.bfloat16), ndim=3)
+            _require(key_cache, "key_cache", dtype=query.dtype, ndim=4, device=dev)
+            _require(value_cache, "value_cache", dtype=query.dtype, ndim=4, device=dev)
+            _require(block_table, "block_table", dtype=torch.int64, ndim=2, device=dev)
+            _require(context_lens, "context_lens", dtype=torch.int64, ndim=1, device=dev)
+            if key_cache.shape != value_cache.shape:
+                raise ValueError("key_cache and value_cache shapes differ")
         nb, hkv, bs, d = key_cache.shape
         if (hkv, bs, d) != (self.num_kv_heads, self.block_size, self.head_dim):
             raise ValueError(f"cache shape {tuple(key_cache.shape)} does not match "
@@ -118,7 +133,8 @@ class PagedAttention:
         if out_dtype not in _DTYPES:
             raise TypeError(f"out_dtype must be float32 or bfloat16, got {out_dtype}")
         if out is None:
-            out = torch.empty((total_q, h, d), dtype=out_dtype, device=dev)
+            out = (torch.empty_like(query) if out_dtype == dtype and type(query) is torch.Tensor
+                   else torch.empty((total_q, h, d), dtype=out_dtype, device=dev))
         else:
             _require(out, "out", dtype=out_dtype, ndim=3, device=dev)
             if tuple(out.shape) != (total_q, h, d):
@@ -129,7 +145,7 @@ class PagedAttention:
             float(scale) if scale else 0.0, _PATHS[path], int(num_splits), int(max_q_len),
             _KV_REUSE[kv_reuse], _SCHEDULES[schedule])
         ctx = context if context is not None else _lib.context(dev.index or 0)
-        ctx.set_stream(torch.cuda.current_stream(dev).cuda_stream)
+        ctx.set_stream(_lib.current_stream(dev.index or 0))
         _lib.check(_lib.lib().kyro_paged_attention_mq(
             ctx.handle, ctypes.byref(params), query.data_ptr(),
             q_start_loc.data_ptr() if q_start_loc is not None else None,

@@ -78,7 +78,7 @@ class PagedKVCache:
                                      block_table.shape[1], nb, _DTYPES[key.dtype],
                                      _DTYPES[key_cache.dtype], int(max_q_len))
         ctx = _lib.context(dev.index or 0)
-        ctx.set_stream(torch.cuda.current_stream(dev).cuda_stream)
+        ctx.set_stream(_lib.current_stream(dev.index or 0))
         ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
         _lib.check(_lib.lib().kyro_paged_kv_append(
             ctx.handle, ctypes.byref(params), ptr(key), ptr(value), ptr(q_start_loc),

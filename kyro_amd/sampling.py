@@ -124,7 +124,7 @@ def sample_tokens_async(logits, temperature, u, *, top_p=None, top_k=None, bias=
         out = torch.empty(B, dtype=torch.int32, device=dev)
     params = _lib.SampleParams(B, V, _lib.KYRO_F32, num_masks)
     ctx = _lib.context(dev.index or 0)
-    ctx.set_stream(torch.cuda.current_stream(dev).cuda_stream)
+    ctx.set_stream(_lib.current_stream(dev.index or 0))
     ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
     _lib.check(_lib.lib().kyro_sample_tokens(
         ctx.handle, ctypes.byref(params), ptr(logits), ptr(temperature), ptr(top_p), ptr(top_k), ptr(u),

@@ -78,7 +78,7 @@ def verify_drafts_async(target_logits, draft_logits, draft_tokens, num_draft, te
         q = torch.empty((B, kmax), dtype=torch.float32, device=dev)
     params = _lib.SpecVerifyParams(B, kmax, V, _lib.KYRO_F32, int(window))
     ctx = _lib.context(dev.index or 0)
-    ctx.set_stream(torch.cuda.current_stream(dev).cuda_stream)
+    ctx.set_stream(_lib.current_stream(dev.index or 0))
     ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
     entry = _lib.lib().kyro_spec_verify_noalloc if allocation_free else _lib.lib().kyro_spec_verify
     _lib.check(entry(
