@@ -85,7 +85,7 @@ struct PfCfg {
 // Copies one slab (16 tokens of one kv head, `base`) into LDS at dst (wave-uniform). V selects the
 // V swizzle. Columns past the head dim (DR < D) repeat the row's last chunk: K's are never read,
 // V's reach only output columns that are not stored.
-template <class C, bool V>
+template <class C, bool V, int POL>
 __device__ __forceinline__ void copy_slab(uint4* dst, const void* base, int lane) {
     const __amdgpu_buffer_rsrc_t r =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, kPfBS * C::CPR * 16, kRawWord3);
@@ -99,7 +99,7 @@ __device__ __forceinline__ void copy_slab(uint4* dst, const void* base, int lane
         int c = cg * C::CW + (slot ^ (V ? C::swv(t) : C::swk(t)));
         if (C::CPR < C::NCH) c = min(c, C::CPR - 1);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst + 64 * e), 16,
-                                                 (t * C::CPR + c) * 16, 0, 0, kLoadCached);
+                                                 (t * C::CPR + c) * 16, 0, 0, POL);
     }
 }
 
@@ -146,7 +146,9 @@ struct PfState {
 // running maximum, so that O^T and l cannot overflow after a much larger score.
 constexpr float kDrop = 30.f;
 
-template <bool BF16, int DR>
+// POL: cache policy of the K/V copies. Streaming where no other row group reads the slabs (a verify
+// step's 72 rows per kv head, 64 sequences of 4096 tokens: 201 us with cached loads, 178 us so).
+template <bool BF16, int DR, int POL>
 __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn_prefill_kernel(PrefillArgs p) {
     using C = PfCfg<BF16, DR>;
     const AttnArgs& a = p.a;
@@ -245,12 +247,12 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
     // Copies tile i: with four slabs wave w takes slab w of K and of V, with two a whole slab.
     auto issue = [&](int i, uint4* k, uint4* v) {
         if constexpr (C::NS == 4) {
-            copy_slab<C, false>(k + wave * C::SLAB, slab_ptr(a.k, i, wave), lane);
-            copy_slab<C, true>(v + wave * C::SLAB, slab_ptr(a.v, i, wave), lane);
+            copy_slab<C, false, POL>(k + wave * C::SLAB, slab_ptr(a.k, i, wave), lane);
+            copy_slab<C, true, POL>(v + wave * C::SLAB, slab_ptr(a.v, i, wave), lane);
         } else if (wave < 2) {
-            copy_slab<C, false>(k + wave * C::SLAB, slab_ptr(a.k, i, wave), lane);
+            copy_slab<C, false, POL>(k + wave * C::SLAB, slab_ptr(a.k, i, wave), lane);
         } else {
-            copy_slab<C, true>(v + (wave - 2) * C::SLAB, slab_ptr(a.v, i, wave - 2), lane);
+            copy_slab<C, true, POL>(v + (wave - 2) * C::SLAB, slab_ptr(a.v, i, wave - 2), lane);
         }
     };
 
@@ -591,7 +593,11 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_combine_kernel(Prefil
 
 template <bool BF16, int DR>
 void launch_prefill_dim(const PrefillArgs& p, hipStream_t stream) {
-    attn_prefill_kernel<BF16, DR><<<dim3((unsigned)((long long)p.list_cap * p.a.Hkv)), kPfThreads, 0, stream>>>(p);
+    const dim3 grid((unsigned)((long long)p.list_cap * p.a.Hkv));
+    // The streaming form is built where prefill_rows sends single row groups.
+    constexpr int kOnce = BF16 && DR == 128 ? kLoadStream : kLoadCached;
+    if (p.a.stream_kv) attn_prefill_kernel<BF16, DR, kOnce><<<grid, kPfThreads, 0, stream>>>(p);
+    else attn_prefill_kernel<BF16, DR, kLoadCached><<<grid, kPfThreads, 0, stream>>>(p);
     if (p.part_cap > 0) {
         constexpr long long kMaxGrid = 2048;
         const long long units = (p.list ? (long long)(p.part_cap / 2 + 1) : (long long)p.a.B * p.a.row_groups) * p.a.Hkv *

@@ -187,7 +187,7 @@ int prefill_splits(long long items, long long most, int num_cus, int wgs_per_cu,
 
 // Work bounds and workspace of a launch of the many-row kernel (prefill_attention.hip). False where
 // a bound passes what one launch carries.
-bool prefill_setup(int num_cus, AttnSetup& s) {
+bool prefill_setup(int num_cus, int kv_reuse, AttnSetup& s) {
     kyro::AttnArgs& a = s.a;
     kyro::PrefillArgs& f = s.pf;
     f.tile_tokens = kyro::prefill_tile_tokens(a.dtype_bf16, a.D);
@@ -195,6 +195,7 @@ bool prefill_setup(int num_cus, AttnSetup& s) {
     f.split_cost = a.dtype_bf16 ? 6 : 2;
     a.rows_per_group = kyro::kPrefillRows;
     a.row_groups = (a.rows_cap + kyro::kPrefillRows - 1) / kyro::kPrefillRows;
+    a.stream_kv = kv_reuse == KYRO_KV_REUSE_STREAM || (kv_reuse == KYRO_KV_REUSE_AUTO && a.row_groups == 1);
     const long long all = (long long)a.B * a.row_groups;
     const long long groups = std::min(all, (long long)a.total_q * a.group / kyro::kPrefillRows + a.B);
     if (all > INT32_MAX) return false;
@@ -324,10 +325,11 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     if (many_rows && mfma_blocks && kyro::prefill_head_dim(p->head_dim, p->dtype == KYRO_BF16) &&
         (p->path == KYRO_ATTN_AUTO || (p->path == KYRO_ATTN_MFMA && mfma_ok)) && p->num_splits <= 0 &&
         p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (long long)p->max_blocks_per_seq * p->block_size < (1ll << 30) &&
-        kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, (long long)p->total_q * group, p->batch_size, p->num_kv_heads)) {
+        kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, (long long)p->total_q * group, p->batch_size, p->num_kv_heads,
+                           (long long)group * max_q_len)) {
         a.ubs = 16;
         a.sub = a.bs / 16;
-        if (prefill_setup(num_cus, s)) return KYRO_OK;
+        if (prefill_setup(num_cus, p->kv_reuse, s)) return KYRO_OK;
         a.ubs = kernel == kyro::ATTN_KERNEL_MFMA ? 16 : p->block_size;
         a.sub = a.bs / a.ubs;
     }

@@ -23,6 +23,8 @@ EDGES = {
     # lengths far apart: the listed schedule, with and without split row groups
     "ragged": ((8, 2), [3000, 90, 700, 17, 1500], [40, 80, 512, 17, 200]),
 }
+# a verify step of 72 rows per kv head: one row group a unit, streaming loads
+EDGES["verify72"] = ((64, 8), [700, 9, 64, 65, 300, 1, 0, 1300] * 2, [9] * 16)
 DIMS = [("bf16", D) for D in (64, 80, 96, 112, 128, 160, 192, 224, 256)] + [("f32", D) for D in (64, 80, 96, 112, 128)]
 
 
@@ -53,6 +55,8 @@ def _takes_many_rows(case):
 @pytest.mark.parametrize("dtype,D", DIMS, ids=lambda x: str(x))
 @pytest.mark.parametrize("name", sorted(EDGES))
 def test_many_rows_parity(gpu, name, dtype, D):
+    if name == "verify72" and (dtype, D) != ("bf16", 128):
+        pytest.skip("these rows take another kernel")
     case = _case(name, dtype, D, block=32 if D % 96 == 0 else 16)
     t = h.attention_tensors(case, gpu)
     exp = h.oracle_attention(case)
@@ -62,7 +66,7 @@ def test_many_rows_parity(gpu, name, dtype, D):
 
 def test_the_edges_reach_the_many_row_kernel():
     taken = [name for name in sorted(EDGES) for dtype, D in (("bf16", 128), ("f32", 64)) if _takes_many_rows(_case(name, dtype, D))]
-    assert taken == [name for name in sorted(EDGES) for _ in range(2)]
+    assert taken == [name for name in sorted(EDGES) for _ in range(1 if name == "verify72" else 2)]
 
 
 @pytest.mark.parametrize("dtype,D,block", [("bf16", 128, 16), ("bf16", 80, 64), ("f32", 64, 32)])
