@@ -28,9 +28,11 @@ ARCH = "gfx950"
 # them to VGPRs in every loop iteration (64 v_accvgpr_read per block pair in the two-tile
 # kernel). In VGPR form those copies go, the kernels need 70-100 fewer registers and the
 # four-tile kernel no longer spills: skewed prefix 151.0 -> 148.0 us, mixed GQA 64/8 396.3 ->
-# 388.0 us, Llama-3-8B attention 167.8 -> 166.7 us. The other head dims' kernels keep the
+# 388.0 us, Llama-3-8B attention 167.8 -> 166.7 us. The f32 kernels of the other head dims add their
+# short product chains up in VGPRs and take the same form (head dim 112, 64 sequences of 1000 tokens,
+# 5 rows, 32/8 heads: 143.6 -> 106.8 us). The other head dims' bf16 kernels keep the
 # default (head dim 160 measured 271.7 -> 298.2 us and 256 432.5 -> 445.7 us in VGPR form).
-EXTRA_FLAGS = {"paged_attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"]}
+EXTRA_FLAGS = {s: ["-mllvm", "-amdgpu-mfma-vgpr-form=true"] for s in ("paged_attention.hip", "paged_attention_hd_f32.hip")}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 

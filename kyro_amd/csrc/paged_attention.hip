@@ -1171,10 +1171,13 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
                                               int nsplit, size_t pb0, size_t pbstep) {
     using Cols = F32Cols<D>;
     constexpr int T = Cols::T;
-    // At the other head dims the kernel stands in for the vector kernel, whose sums are trees: four
-    // chains per score and one per block and output keep its error against 64 bits (16 sequences of
-    // 300-3000 tokens, head dim 64: 2.13e-7 in the vector kernel, 1.91e-7 here). That batch went
-    // from 143 to 31.6 us: the vector kernel spends a shuffle tree per row and token.
+    // At the other head dims the kernel stands in for the vector kernel, whose sums are trees: chains of 8
+    // additions in a score and of 4 in a block's output, added up in trees, and weights taken from the
+    // distance to the maximum keep its error against 64 bits at or below the vector kernel's (32/8 heads,
+    // one row, head dims 64 / 80 / 96 / 112, 1e-7: contexts of 16 tokens 1.11 1.18 1.20 1.16 here, 1.13
+    // 1.18 1.25 1.19 there; of 1000 1.65 1.77 1.83 1.74 and 1.85 1.94 2.02 1.95; four chains per score
+    // and one per output: 1.27 1.39 1.44 1.42 at 16). 16 sequences of 300-3000 tokens, head dim 64: 143
+    // -> 32 us; the vector kernel spends a shuffle tree per row and token.
     constexpr bool kShort = D != kMfmaD;
     constexpr int RW = NTW * 16;
     constexpr int WPH = kWaves / HP;
@@ -1230,18 +1233,34 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
             f32x4 S[NTW];
 #pragma unroll
             for (int nt = 0; nt < NTW; ++nt) {
-                constexpr int NC = kShort ? 4 : 1;
-                f32x4 acc[NC];
+                if constexpr (kShort) {
+                    // Chains of 8 additions over 32 dims, then a tree.
+                    f32x4 part[(T + 1) / 2];
 #pragma unroll
-                for (int x = 0; x < NC; ++x) acc[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    for (int s = 0; s < T; s += 2) {
+                        f32x4 acc[4];
 #pragma unroll
-                for (int s = 0; s < T; ++s)
+                        for (int e = 0; e < 4; ++e) {
+                            acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4_get(kv.k[s], e), f4_get(qB[nt][s], e),
+                                                                          f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                            if (s + 1 < T)
+                                acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4_get(kv.k[s + 1], e),
+                                                                              f4_get(qB[nt][s + 1], e), acc[e], 0, 0, 0);
+                        }
+                        part[s / 2] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+                    }
+                    if constexpr (T <= 4) S[nt] = part[0] + part[1];
+                    else if constexpr (T <= 6) S[nt] = (part[0] + part[1]) + part[2];
+                    else S[nt] = (part[0] + part[1]) + (part[2] + part[3]);
+                } else {
+                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        acc[e % NC] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4_get(kv.k[s], e), f4_get(qB[nt][s], e),
-                                                                           acc[e % NC], 0, 0, 0);
-                if constexpr (kShort) S[nt] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-                else S[nt] = acc[0];
+                    for (int s = 0; s < T; ++s)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(f4_get(kv.k[s], e), f4_get(qB[nt][s], e), acc, 0, 0, 0);
+                    S[nt] = acc;
+                }
             }
             const bool full = blk >= 0 && (pb + 1) * kMfmaBS <= full_vis;
             if (!full) {
@@ -1268,13 +1287,15 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
                 }
                 float mx = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
                 mx = max_over_rows(mx);
-                const float m_new = fmaxf(m[nt], mx * c);
+                // kShort: m stays unscaled until the waves merge, so that a weight's error is relative to
+                // the distance from the maximum and the largest weight is exactly 1.
+                const float m_new = fmaxf(m[nt], kShort ? mx : mx * c);
                 const float mref = (m_new == kNegInf) ? 0.f : m_new;
-                const float alpha = fast_exp2(m[nt] - mref);
+                const float alpha = fast_exp2(kShort ? (m[nt] - mref) * c : m[nt] - mref);
                 float ps = 0.f;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    pv[nt][e] = fast_exp2(__builtin_fmaf(sv[e], c, -mref));
+                    pv[nt][e] = fast_exp2(kShort ? (sv[e] - mref) * c : __builtin_fmaf(sv[e], c, -mref));
                     ps += pv[nt][e];
                 }
                 lsum[nt] = lsum[nt] * alpha + ps;
@@ -1289,11 +1310,12 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
                 for (int dt = 0; dt < T; ++dt)
 #pragma unroll
                     for (int nt = 0; nt < NTW; ++nt) {
-                        f32x4 add = {0.f, 0.f, 0.f, 0.f};
+                        f32x4 add[4];
 #pragma unroll
                         for (int q = 0; q < 4; ++q)
-                            add = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.v[q][dt], pv[nt][q], add, 0, 0, 0);
-                        O[dt][nt] += add;
+                            add[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.v[q][dt], pv[nt][q],
+                                                                          f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                        O[dt][nt] += (add[0] + add[1]) + (add[2] + add[3]);
                     }
             } else {
 #pragma unroll
@@ -1369,7 +1391,15 @@ __device__ __forceinline__ void mfma_item_f32(const AttnArgs& a, Frame<NTW * 16,
             float M = fr.m[0][n];
 #pragma unroll
             for (int w = 1; w < WPH; ++w) M = fmaxf(M, fr.m[w][n]);
-            f[nt] = (m[nt] == kNegInf) ? 0.f : fast_exp2(m[nt] - M);
+            if constexpr (kShort) {
+                // Parts of a split row are weighed by the rounded scaled maximum: relative to it then.
+                const float Mc = M * c;
+                f[nt] = m[nt] == kNegInf ? 0.f
+                                         : fast_exp2(nsplit > 1 ? __builtin_fmaf(m[nt], c, -Mc) : (m[nt] - M) * c);
+                M = Mc;
+            } else {
+                f[nt] = (m[nt] == kNegInf) ? 0.f : fast_exp2(m[nt] - M);
+            }
             if (g == 0) {
                 fr.l[wp][n] = lsum[nt] * f[nt];
                 if (wp == 0) fr.mx[n] = M;

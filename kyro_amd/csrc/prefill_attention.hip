@@ -70,7 +70,13 @@ struct PfCfg {
     static constexpr int TK = prefill_tile_tokens(BF16, DR);
     static constexpr int NS = TK / kPfBS;            // slabs of a tile
     static constexpr int TT = TK / 32;               // 32-token tiles of S^T
-    static constexpr int SC = DR > 96 ? 2 : 8;       // f32: accumulators per score (what registers allow)
+    // f32 head dims where the kernel stands in for the vector kernel, whose sums are trees: short chains
+    // of additions (8 in a score, 4 in a tile's O^T += V^T P^T) that are added up in two halves. The error
+    // against 64 bits is then level with the vector kernel's over 33 to 4000 tokens (prompts of 200 tokens,
+    // head dims 64 / 80 / 96 / 112, 1e-7: 1.15 1.22 1.24 1.23 here, 1.16 1.22 1.26 1.23 there; with two
+    // chains per score, as at 128, 1.82 at 112). At head dim 128 two long chains per score and one per
+    // output are already closer than the one-block kernel's single chain (1.89 against 2.80).
+    static constexpr bool TREE = !BF16 && DR < 128;
     // K rows: chunk c of token t sits in slot c ^ swk(t) of its column group, so that the 16
     // tokens of an operand read (same c) spread over all banks.
     __device__ static constexpr int swk(int t) { return t * CW / 16; }
@@ -314,27 +320,32 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
             }
             __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
         } else {
-            // Several short chains per score instead of one of DR / 2 sequential additions, in step with
-            // the vector kernel's tree sums (head dim 64, error against 64 bits: 3.5e-7 with one chain
-            // here and per output below, 1.6e-7 so and in the vector kernel).
             static_assert(BF16 || C::TT == 1, "one 32-token tile of scores at a time");
-            f32x16 part[C::SC];
+            f32x16 half[2];
 #pragma unroll
-            for (int y = 0; y < C::SC; ++y)
+            for (int y = 0; y < 2; ++y)
 #pragma unroll
-                for (int x = 0; x < 16; ++x) part[y][x] = 0.f;
+                for (int x = 0; x < 16; ++x) half[y][x] = 0.f;
 #pragma unroll
             for (int s = 0; s < C::KS; ++s) {
                 const f32x4 kf = __builtin_bit_cast(f32x4, k_operand(s, 0)), qf = __builtin_bit_cast(f32x4, q[s]);
+                if constexpr (C::TREE) {
+                    f32x16 chain;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    f32x16& to = part[(4 * s + e) % C::SC];
-                    to = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[e], to, 0, 0, 0);
+                    for (int x = 0; x < 16; ++x) chain[x] = 0.f;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) chain = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[e], chain, 0, 0, 0);
+                    f32x16& to = half[s / (C::KS / 2)];
+                    if (s % (C::KS / 2) == 0) to = chain;
+                    else to += chain;
+                    if (s % 2) __builtin_amdgcn_sched_barrier(0);  // two chains in flight, no more (registers)
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        half[e % 2] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[e], half[e % 2], 0, 0, 0);
                 }
             }
-            if constexpr (C::SC == 8)
-                S[0] = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
-            else S[0] = part[0] + part[1];
+            S[0] = half[0] + half[1];
         }
         if (t0 + C::TK > wave_lo || tbad) {
 #pragma unroll
@@ -355,12 +366,19 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
             const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
             mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
         }
-        mx *= c;
-        st.top = fmaxf(st.top, mx);
-        float m_new = fmaxf(mx, st.top - kDrop);
-        if constexpr (!BF16) m_new = ceilf(m_new);  // the rescale is then by a power of two: exact
-        // -inf - -inf (nothing visible yet) would be NaN; O^T and l are 0 then.
-        const float alpha = st.m == kNegInf ? 0.f : fast_exp2(st.m - m_new);
+        float m_new, alpha;
+        if constexpr (BF16) {
+            mx *= c;
+            st.top = fmaxf(st.top, mx);
+            m_new = fmaxf(mx, st.top - kDrop);
+            // -inf - -inf (nothing visible yet) would be NaN; O^T and l are 0 then.
+            alpha = st.m == kNegInf ? 0.f : fast_exp2(st.m - m_new);
+        } else {
+            // The running maximum, unscaled until the state is stored: a weight's error is relative to
+            // its distance from the maximum, and the largest weight is exactly 1.
+            m_new = fmaxf(st.m, mx);
+            alpha = st.m == kNegInf ? 0.f : fast_exp2((st.m - m_new) * c);
+        }
 #pragma unroll
         for (int dt = 0; dt < C::DT; ++dt) st.o[dt] *= alpha;
         st.l *= alpha;
@@ -372,7 +390,7 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
             float pt[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int x = 0; x < 16; ++x) {
-                S[tt][x] = fast_exp2(__builtin_fmaf(S[tt][x], c, -mref));
+                S[tt][x] = fast_exp2(BF16 ? __builtin_fmaf(S[tt][x], c, -mref) : (S[tt][x] - mref) * c);
                 pt[x % 4] += S[tt][x];
             }
             ps += (pt[0] + pt[1]) + (pt[2] + pt[3]);
@@ -403,28 +421,40 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
                     }
                 }
         } else {
-            // A tile's products are summed on their own and then added: the chain of additions into
-            // O^T is one per tile instead of one per two tokens.
-            constexpr int W = C::DT % 2 ? 1 : 2;  // column tiles side by side
+            // A tile's products are summed on their own and then added: the chain of additions into O^T
+            // is one per tile instead of one per two tokens.
+            constexpr int W = C::TREE ? 1 : 2;    // column tiles side by side
+            constexpr int NC = C::TREE ? 8 : 1;   // chains of a tile's 16 products
 #pragma unroll
             for (int d0 = 0; d0 < C::DT; d0 += W) {
-                f32x16 add[W];
+                f32x16 half[2][W];
 #pragma unroll
-                for (int w = 0; w < W; ++w)
+                for (int y = 0; y < NC; ++y) {
+                    f32x16 chain[W];
 #pragma unroll
-                    for (int x = 0; x < 16; ++x) add[w][x] = 0.f;
+                    for (int w = 0; w < W; ++w)
 #pragma unroll
-                for (int x = 0; x < 16; ++x)
+                        for (int x = 0; x < 16; ++x) chain[w][x] = 0.f;
+#pragma unroll
+                    for (int x = y * (16 / NC); x < (y + 1) * (16 / NC); ++x)
+#pragma unroll
+                        for (int w = 0; w < W; ++w) {
+                            const int dt = d0 + w;
+                            const float vv = *reinterpret_cast<const float*>(
+                                vb + vaddr32 + (x / 8) * (C::SLAB * 16) + (8 * dt / C::CW) * kGroupBytes +
+                                (8 * ((x / 4) % 2) + x % 4) * (C::CW * 16) + (8 * dt % C::CW) * 16);
+                            chain[w] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, S[0][x], chain[w], 0, 0, 0);
+                        }
 #pragma unroll
                     for (int w = 0; w < W; ++w) {
-                        const int dt = d0 + w;
-                        const float vv = *reinterpret_cast<const float*>(
-                            vb + vaddr32 + (x / 8) * (C::SLAB * 16) + (8 * dt / C::CW) * kGroupBytes +
-                            (8 * ((x / 4) % 2) + x % 4) * (C::CW * 16) + (8 * dt % C::CW) * 16);
-                        add[w] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, S[0][x], add[w], 0, 0, 0);
+                        f32x16& to = half[2 * y / NC][w];
+                        if (2 * y % NC == 0) to = chain[w];
+                        else to += chain[w];
                     }
+                    if (C::TREE && y % 2) __builtin_amdgcn_sched_barrier(0);
+                }
 #pragma unroll
-                for (int w = 0; w < W; ++w) st.o[d0 + w] += add[w];
+                for (int w = 0; w < W; ++w) st.o[d0 + w] += C::TREE ? half[0][w] + half[1][w] : half[0][w];
             }
         }
     };
@@ -470,7 +500,7 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
     }
 
     if (n >= si.rows) return;
-    const float L = st.l + __shfl_xor(st.l, 32, 64);
+    float L = st.l + __shfl_xor(st.l, 32, 64);
     if (part < 0) {
         const float inv = L > 0.f ? 1.f / L : 0.f;
         const size_t row = out_row(a, si, n);
@@ -487,6 +517,15 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
     }
     // A part's state: m and l by row, O^T in the order the lanes hold it (whole 1 KiB stores).
     const size_t wv = ((size_t)part * a.Hkv + kvh) * kPfWaves + wave;
+    if constexpr (!BF16) {
+        // Relative to the rounded scaled maximum that the merge weighs parts by.
+        const float m = st.m * c;
+        const float f = st.m == kNegInf ? 1.f : fast_exp2(__builtin_fmaf(st.m, c, -m));
+        st.m = m;
+        L *= f;
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt) st.o[dt] *= f;
+    }
     if (h == 0) {
         a.ws_m[wv * 32 + col] = st.m;
         a.ws_l[wv * 32 + col] = L;

@@ -55,6 +55,29 @@ def oracle_attention(case: wl.AttentionCase, seqs=None, causal=True) -> dict:
     return res
 
 
+def attention_float64(case: wl.AttentionCase) -> torch.Tensor:
+    """Causal attention of every query row in 64 bits, [total_q, H, D], on the host."""
+    H, Hkv, D = case.num_heads, case.num_kv_heads, case.head_dim
+    cast = (lambda x: wl.bf16_bits_to_f32(x)) if case.dtype == "bf16" else np.asarray
+    out = torch.zeros(case.query.shape, dtype=torch.float64)
+    for b in range(case.batch):
+        ctx = int(case.context_lens[b])
+        q0, q1 = int(case.q_start_loc[b]), int(case.q_start_loc[b + 1])
+        n = q1 - q0
+        if n == 0 or ctx == 0:
+            continue
+        ids = case.block_table[b, :-(-ctx // case.block_size)]
+        k, v = (torch.from_numpy(cast(x[ids])).double().transpose(0, 1).reshape(Hkv, -1, D)[:, :ctx]
+                for x in (case.key_cache, case.value_cache))
+        q = torch.from_numpy(cast(case.query[q0:q1])).double().view(n, Hkv, H // Hkv, D).permute(1, 2, 0, 3)
+        s = torch.matmul(q.reshape(Hkv, -1, D), k.transpose(1, 2)).view(Hkv, H // Hkv, n, ctx) / D ** 0.5
+        seen = torch.arange(ctx) <= ctx - n + torch.arange(n).view(-1, 1)
+        p = torch.softmax(s.masked_fill(~seen, float("-inf")), -1).nan_to_num()  # a row that sees nothing: 0
+        o = torch.matmul(p.view(Hkv, -1, ctx), v).view(Hkv, H // Hkv, n, D)
+        out[q0:q1] = o.permute(2, 0, 1, 3).reshape(n, H, D)
+    return out
+
+
 def assert_attention_close(out: torch.Tensor, case: wl.AttentionCase, expected: dict, atol: float):
     got = out.float().cpu().numpy()
     worst = 0.0

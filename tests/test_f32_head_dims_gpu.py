@@ -50,3 +50,47 @@ def test_f32_head_dims_stay_refused_by_name(gpu):
         with pytest.raises(kyro_amd.KyroError):
             attn.forward(t["query"], t["key_cache"], t["value_cache"], t["block_table"], t["context_lens"],
                          q_start_loc=t["q_start_loc"], **kw)
+
+
+# (heads, kv heads, sequences, query rows, context): contexts short enough that rounding of the scores
+# and of the first sums shows, one and two row tiles, and prompts (the many-row kernel).
+PRECISION = {
+    "decode": (32, 8, 48, 1, 16),
+    "mha": (16, 16, 48, 1, 64),
+    "verify": (32, 8, 16, 5, 33),
+    "prompt": (16, 4, 4, 64, 64),
+    "long_prompt": (16, 4, 2, 200, 200),
+    "chunk": (16, 4, 2, 64, 500),
+}
+
+
+@pytest.mark.parametrize("D", [64, 80, 96, 112])
+@pytest.mark.parametrize("name", sorted(PRECISION))
+def test_f32_error_against_64_bits_is_the_vector_kernels(gpu, name, D):
+    """Automatic choice must not cost precision over the vector kernel's tree sums: the same 32-bit
+    operations in chains no deeper give the same error up to sampling. The ratio of two error norms over
+    50 thousand values or more scatters by about 1%, and a few operations more or fewer in either kernel
+    move it by another 2%; chains twice as long make it 1.08 or more at every shape but "chunk"."""
+    H, Hkv, B, q, ctx = PRECISION[name]
+    case = wl.make_attention_case(context_lens=[ctx] * B, q_lens=[q] * B, num_heads=H, num_kv_heads=Hkv, head_dim=D,
+                                  dtype="f32", seed=D + ctx)
+    t = h.attention_tensors(case, gpu)
+    attn = kyro_amd.PagedAttention(case.block_size, H, D, Hkv)
+    exact = h.attention_float64(case)
+    err = {}
+    for path in ("auto", "vector"):
+        out = attn.forward(t["query"], t["key_cache"], t["value_cache"], t["block_table"], t["context_lens"],
+                           q_start_loc=t["q_start_loc"], path=path)
+        err[path] = float((out.cpu().double() - exact).norm() / exact.norm())
+    assert err["auto"] <= 1.05 * err["vector"], err
+
+
+@pytest.mark.parametrize("D", [64, 112])
+def test_f32_context_of_one_token_is_its_value(gpu, D):
+    case = wl.make_attention_case(context_lens=[1] * 8, q_lens=[1] * 8, num_heads=8, num_kv_heads=2, head_dim=D,
+                                  dtype="f32", seed=D)
+    t = h.attention_tensors(case, gpu)
+    out = kyro_amd.PagedAttention(16, 8, D, 2).forward(t["query"], t["key_cache"], t["value_cache"], t["block_table"],
+                                                       t["context_lens"], q_start_loc=t["q_start_loc"])
+    v = t["value_cache"][t["block_table"][:, 0], :, 0, :]
+    assert torch.equal(out, v.repeat_interleave(4, dim=1))
