@@ -143,14 +143,15 @@ struct PfState {
     float top;        // running maximum
     float l;          // this lane's share of the row sum
 };
-// The weights of a tile are relative to the tile's own maximum, so that the largest is 1, which bf16
-// holds exactly. That costs a rescale of O^T per tile (four 2048-token prompts, head dim 128:
-// 169.6 us with a reference that may lag the maximum by 2^8 and so hardly ever moves, 178 so) and
-// lowers the error against 64 bits from 2.09e-3 with the lagging reference and 2.03e-3 with one
-// running maximum to 1.98e-3, where the kernels that stream K/V per wave have 1.97e-3 (contexts of
-// 700-8000 tokens: 2.33e-3, 2.23e-3, 2.09e-3, 2.19e-3). The reference stays within 2^kDrop of the
-// running maximum, so that O^T and l cannot overflow after a much larger score.
-constexpr float kDrop = 30.f;
+// bf16: the reference of a tile's weights is the running maximum, moved up by less than 1 so that it lies
+// a whole number above the tile's own maximum: the tile's largest weight is then a power of two, which
+// bf16 holds exactly, and no weight passes 1, so that O^T and l stay within the sums of |V| and of ones
+// whatever the order of the scores (a reference that may fall 2^30 below it overflows O^T for |V| above
+// 1e29; 166.1 against 167.6 us for four 2048-token prompts, head dim 128). Against a reference that lags
+// the maximum by up to 2^8 and so hardly ever moves, the rescale of O^T per tile costs 5% of that time
+// and lowers the error against 64 bits from 2.09e-3 (2.03e-3 with the plain running maximum) to 1.98e-3,
+// where the kernels that stream K/V per wave have 1.97e-3 (contexts of 700-8000 tokens: 2.33e-3,
+// 2.23e-3, 2.09e-3, 2.19e-3).
 
 // POL: cache policy of the K/V copies. Streaming where no other row group reads the slabs (a verify
 // step's 72 rows per kv head, 64 sequences of 4096 tokens: 201 us with cached loads, 178 us so).
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
         if constexpr (BF16) {
             mx *= c;
             st.top = fmaxf(st.top, mx);
-            m_new = fmaxf(mx, st.top - kDrop);
+            m_new = mx == kNegInf ? st.top : mx + ceilf(st.top - mx);
             // -inf - -inf (nothing visible yet) would be NaN; O^T and l are 0 then.
             alpha = st.m == kNegInf ? 0.f : fast_exp2(st.m - m_new);
         } else {

@@ -101,6 +101,25 @@ def test_many_rows_after_a_much_larger_score(gpu):
     h.assert_attention_close(out, case, h.oracle_attention(case), 4 * h.ATOL_BF16)  # values up to 4
 
 
+@pytest.mark.parametrize("dtype,D", [("bf16", 128), ("bf16", 64), ("f32", 64), ("f32", 128)])
+def test_many_rows_large_values_after_a_much_larger_score(gpu, dtype, D):
+    """The same with values of 1e30: every weighted sum is far below the type's largest value, and so must
+    be whatever the kernel holds on the way. (bf16: three roundings of 2^-9; sums of like sign aside, the
+    error of an output is bounded by 4 * 2^-9 of the largest value.)"""
+    case = _case("ragged", dtype, D, seed=6)
+    t = h.attention_tensors(case, gpu)
+    first = t["block_table"][:, 0]
+    t["key_cache"][first, :, 0, :] = 40.0 * torch.sign(t["key_cache"][first, :, 0, :])
+    t["value_cache"] *= 1e30
+    for x in ("key_cache", "value_cache"):
+        host = t[x].cpu()
+        setattr(case, x, host.view(torch.int16).numpy().view(np.uint16) if dtype == "bf16" else host.numpy())
+    out = _attention(case).forward(*_args(t), q_start_loc=t["q_start_loc"]).cpu().double()
+    assert torch.isfinite(out).all()
+    exact = h.attention_float64(case)
+    assert float((out - exact).abs().max()) <= (4 * 2.0 ** -9 if dtype == "bf16" else 1e-4) * float(t["value_cache"].abs().max())
+
+
 def test_many_rows_errors_latch(gpu):
     """A bad block id, a context longer than its table and rows out of order are reported; the
     sequences without a fault are computed as before."""
