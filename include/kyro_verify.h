@@ -83,7 +83,10 @@ int kyro_ctx_set_stream(kyro_ctx ctx, void* hip_stream);
  * A call that needs more arena than the context holds synchronises the stream, frees the arena
  * and allocates a larger one; kernels captured into a HIP graph before that point would then
  * address freed memory. A caller that captures calls into a graph should reserve the largest
- * arena those calls need first (or re-capture after a growth). The balanced attention schedule
+ * arena those calls need first (or re-capture after a growth). An attention call that is captured
+ * while the arena is too small for the form automatic choice prefers (many-row kernel, short
+ * chunks) takes one that needs no more than the arena holds, where there is one, and is refused
+ * (KYRO_EINVAL, naming the bytes) where there is none. The balanced attention schedule
  * and the one-launch decode sampler (kyro_sample_tokens without processors, top-k or top-p) also
  * keep small counters in the context that every launch returns to zero, so their launches replay
  * from a graph as they run eagerly. */

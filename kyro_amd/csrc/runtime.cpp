@@ -234,8 +234,19 @@ bool prefill_setup(int num_cus, int kv_reuse, AttnSetup& s) {
     return true;
 }
 
+// Forms of a launch that automatic choice may take beside the grid and the balanced schedule.
+enum AttnForms : int {
+    FORM_MANY_ROWS = 1,     // the many-row kernel
+    FORM_SHORT_CHUNKS = 2,  // the grid in short chunks
+    FORM_F32_DIMS = 4,      // the MFMA kernel for f32 caches at head dims other than 128
+    FORMS_ALL = 7,
+    // None of them: what takes the least scratch (a table of up to 4096 tokens takes none with at least
+    // one workgroup a CU), for a graph capture whose arena holds no more.
+    FORMS_LEAST_SCRATCH = 0
+};
+
 int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int num_cus, AttnSetup& s,
-                    int chunk_quarters = kyro::kPlanChunkQuarters, bool many_rows = true) {
+                    int chunk_quarters = kyro::kPlanChunkQuarters, int forms = FORMS_ALL) {
     if (!p) return fail(KYRO_EINVAL, "paged_attention: params is null");
     if (p->block_size <= 0 || p->num_heads <= 0 || p->head_dim <= 0 || p->num_kv_heads <= 0)
         return fail(KYRO_EINVAL, "paged_attention: block_size/num_heads/head_dim/num_kv_heads must be > 0");
@@ -293,7 +304,7 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
         // MFMA wherever it applies, one query row per kv head included: the kernel is
         // memory-bound, so padding rows to a 16-row tile costs nothing measurable (MHA decode,
         // 1 row per kv head: 67 us against the vector kernel's 207 us).
-        const bool f32_auto = mfma_blocks && p->dtype == KYRO_F32 && kyro::mfma_f32_auto_dim(p->head_dim) &&
+        const bool f32_auto = (forms & FORM_F32_DIMS) && mfma_blocks && p->dtype == KYRO_F32 && kyro::mfma_f32_auto_dim(p->head_dim) &&
                               p->schedule != KYRO_ATTN_SCHEDULE_BALANCED;
         kernel = mfma_ok || f32_auto ? kyro::ATTN_KERNEL_MFMA : kyro::ATTN_KERNEL_VECTOR;
     }
@@ -322,7 +333,7 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     const double scale = p->scale > 0 ? (double)p->scale : 1.0 / std::sqrt((double)p->head_dim);
     a.scale_log2 = (float)(scale * 1.4426950408889634);
     a.units = p->batch_size * p->num_kv_heads;
-    if (many_rows && mfma_blocks && kyro::prefill_head_dim(p->head_dim, p->dtype == KYRO_BF16) &&
+    if ((forms & FORM_MANY_ROWS) && mfma_blocks && kyro::prefill_head_dim(p->head_dim, p->dtype == KYRO_BF16) &&
         (p->path == KYRO_ATTN_AUTO || (p->path == KYRO_ATTN_MFMA && mfma_ok)) && p->num_splits <= 0 &&
         p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (long long)p->max_blocks_per_seq * p->block_size < (1ll << 30) &&
         kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, (long long)p->total_q * group, p->batch_size, p->num_kv_heads,
@@ -405,8 +416,8 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     // with 94 at 32/8 heads. Short bf16 contexts that took one launch before (up to 496 tokens) keep
     // it: 300 tokens 11.9 us, 14.6 in chunks (f32 20.1 and 14.8).
     bool short_chunks = false;
-    if (kernel == kyro::ATTN_KERNEL_MFMA && p->num_splits == 0 && p->schedule == KYRO_ATTN_SCHEDULE_AUTO &&
-        (splits > 1 || p->dtype == KYRO_F32 || p->head_dim > 128)) {
+    if ((forms & FORM_SHORT_CHUNKS) && kernel == kyro::ATTN_KERNEL_MFMA && p->num_splits == 0 &&
+        p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (splits > 1 || p->dtype == KYRO_F32 || p->head_dim > 128)) {
         const long long groups = (long long)a.ugroups * a.row_groups;
         const bool narrow = a.row_groups == 1 && p->head_dim <= 128;
         for (int c : {8, 16, 32}) {
@@ -766,11 +777,27 @@ int kyro_paged_attention_mq(kyro_ctx ctx, const kyro_paged_attention_params* p, 
         AttnSetup s;
         // The many-row kernel copies cache rows to LDS 16 bytes at a time.
         const bool aligned = ((reinterpret_cast<uintptr_t>(key_cache) | reinterpret_cast<uintptr_t>(value_cache)) & 15) == 0;
-        if (int rc = attention_setup(p, q_start_loc != nullptr, ctx->num_cus, s, kyro::kPlanChunkQuarters, aligned))
+        if (int rc = attention_setup(p, q_start_loc != nullptr, ctx->num_cus, s, kyro::kPlanChunkQuarters,
+                                     aligned ? FORMS_ALL : FORMS_ALL & ~FORM_MANY_ROWS))
             return rc;
         if (s.empty) return KYRO_OK;
         if (!query || !key_cache || !value_cache || !block_table || !context_lens || !out)
             return fail(KYRO_EINVAL, "paged_attention: null device pointer");
+        DeviceGuard dg(ctx->device);
+        KYRO_HIP(dg.status);
+        if (s.ws_bytes > ctx->arena_bytes) {
+            // While the stream captures a graph the arena cannot grow: a form that needs no more than
+            // it holds takes the call then.
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            KYRO_HIP(hipStreamIsCapturing(ctx->stream, &cap));
+            if (cap != hipStreamCaptureStatusNone) {
+                AttnSetup lean;
+                if (int rc = attention_setup(p, q_start_loc != nullptr, ctx->num_cus, lean, kyro::kPlanChunkQuarters,
+                                             FORMS_LEAST_SCRATCH))
+                    return rc;
+                if (lean.ws_bytes <= ctx->arena_bytes) s = lean;
+            }
+        }
         kyro::AttnArgs& a = s.a;
         a.q = query;
         a.q_start = q_start_loc;
@@ -779,8 +806,6 @@ int kyro_paged_attention_mq(kyro_ctx ctx, const kyro_paged_attention_params* p, 
         a.table = block_table;
         a.ctx_lens = context_lens;
         a.out = out;
-        DeviceGuard dg(ctx->device);
-        KYRO_HIP(dg.status);
         if (s.ws_bytes) {
             if (int rc = ensure_arena(ctx, s.ws_bytes)) return rc;
             attention_workspace(s, static_cast<char*>(ctx->arena));
@@ -810,7 +835,9 @@ int kyro_paged_attention_workspace(kyro_ctx ctx, const kyro_paged_attention_para
         *bytes = s.ws_bytes;
         if (s.kernel == kyro::ATTN_KERNEL_PREFILL) {  // caches that are not 16-byte aligned take another kernel
             AttnSetup other;
-            if (int rc = attention_setup(p, has_q_start_loc != 0, cus, other, kyro::kPlanChunkQuarters, false)) return rc;
+            if (int rc = attention_setup(p, has_q_start_loc != 0, cus, other, kyro::kPlanChunkQuarters,
+                                         FORMS_ALL & ~FORM_MANY_ROWS))
+                return rc;
             *bytes = std::max(*bytes, other.ws_bytes);
         }
         return KYRO_OK;

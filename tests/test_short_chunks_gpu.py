@@ -51,3 +51,38 @@ def test_short_chunks_parity(gpu, dtype, H, Hkv, D, ctx, ql):
     out = attn.forward(t["query"], t["key_cache"], t["value_cache"], t["block_table"], t["context_lens"],
                        q_start_loc=t["q_start_loc"])
     h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,H,Hkv,D,ctx,ql", [
+    ("bf16", 64, 8, 128, [4000] + [300, 64, 9] * 21, [9] * 64),  # the many-row kernel's list and parts
+    ("f32", 32, 8, 64, [300, 17, 0, 260] * 2, [1] * 8),      # short chunks
+    ("f32", 32, 8, 128, [300, 17, 0, 260], [1] * 4),
+    ("bf16", 8, 8, 256, [300, 17, 0, 260], [1] * 4),
+])
+def test_capture_without_a_reserve_takes_a_form_without_scratch(gpu, dtype, H, Hkv, D, ctx, ql):
+    """Forms chosen for speed alone need scratch at these shapes. A graph captured on a context whose arena
+    is empty takes the form that needs none."""
+    from kyro_amd import _lib
+
+    case = wl.make_attention_case(context_lens=ctx, q_lens=ql, num_heads=H, num_kv_heads=Hkv, head_dim=D, dtype=dtype,
+                                  seed=D + len(ctx))
+    t = h.attention_tensors(case, gpu)
+    attn = kyro_amd.PagedAttention(16, H, D, Hkv)
+    args = (t["query"], t["key_cache"], t["value_cache"], t["block_table"], t["context_lens"])
+    context = _lib.Context(gpu.index or 0)
+    kw = dict(q_start_loc=t["q_start_loc"], max_q_len=max(ql), context=context)
+    s = torch.cuda.Stream(gpu)
+    with torch.cuda.stream(s):  # binds the context to s; one split takes no scratch
+        out = attn.forward_async(*args, num_splits=1, schedule="grid", **kw)
+    context.sync()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        attn.forward_async(*args, out=out, **kw)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32)
+    del g
+    context.sync()
