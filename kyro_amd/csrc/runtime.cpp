@@ -333,11 +333,12 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     const double scale = p->scale > 0 ? (double)p->scale : 1.0 / std::sqrt((double)p->head_dim);
     a.scale_log2 = (float)(scale * 1.4426950408889634);
     a.units = p->batch_size * p->num_kv_heads;
+    // Rows the sequences can bring: padding rows of q belong to none.
+    const long long rows = std::min<long long>(p->total_q, (long long)p->batch_size * max_q_len) * group;
     if ((forms & FORM_MANY_ROWS) && mfma_blocks && kyro::prefill_head_dim(p->head_dim, p->dtype == KYRO_BF16) &&
         (p->path == KYRO_ATTN_AUTO || (p->path == KYRO_ATTN_MFMA && mfma_ok)) && p->num_splits <= 0 &&
         p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (long long)p->max_blocks_per_seq * p->block_size < (1ll << 30) &&
-        kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, (long long)p->total_q * group, p->batch_size, p->num_kv_heads,
-                           (long long)group * max_q_len)) {
+        kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, rows, p->batch_size, p->num_kv_heads, (long long)group * max_q_len)) {
         a.ubs = 16;
         a.sub = a.bs / 16;
         if (prefill_setup(num_cus, p->kv_reuse, s)) return KYRO_OK;
