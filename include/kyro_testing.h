@@ -19,6 +19,14 @@ extern "C" {
  * KYRO_EINVAL. Returns the previous cap. */
 int64_t kyro_testing_set_plan_slot_cap(int64_t cap);
 
+struct kyro_paged_attention_params;
+
+/* Tiles of a part that the many-row attention kernel gives the row groups of a sequence of `ctx` tokens in a
+ * call of these params (256 CUs), and the most parts of one in *splits; 0 where the kernel lists its work
+ * on the device, negative where the call does not take that kernel. No device call. */
+int kyro_testing_prefill_part_tiles(const struct kyro_paged_attention_params* params, int has_q_start_loc,
+                                    int64_t ctx, int* splits);
+
 #ifdef __cplusplus
 }
 #endif

@@ -145,6 +145,8 @@ _SIGNATURES = {
     "kyro_ngram_draft": ([_P, _P, ctypes.c_int32, ctypes.c_int32, _P, _P, _P, _P], ctypes.c_int),
     # include/kyro_testing.h
     "kyro_testing_set_plan_slot_cap": ([ctypes.c_int64], ctypes.c_int64),
+    "kyro_testing_prefill_part_tiles": ([ctypes.POINTER(PagedAttentionParams), ctypes.c_int, ctypes.c_int64,
+                                         ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
 }
 
 

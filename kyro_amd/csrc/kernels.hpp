@@ -227,12 +227,23 @@ struct PrefillArgs {
     int* head;        // {list entries, split row groups}
     int list_cap;     // entries the workspace holds
     int part_cap;     // parts (partial states per kv head) it holds; 0: row groups are not split
-    int splits;       // without a list: parts of a row group at most, part s the tiles from s * chunk on
-    int chunk;
+    int splits;       // without a list: parts of a row group at most (prefill_part_tiles)
+    unsigned splits_magic;  // 2^32 / splits + 1: exact quotients of numbers below 2^25 (at most 64 splits)
+    int least_part, whole_tiles;
     int tile_tokens;  // prefill_tile_tokens
     int slots;        // workgroups the device runs at once
     int split_cost;   // tiles a workgroup computes in the time that parking and merging one part takes
 };
+
+// Without a list: tiles of a part of a sequence's row groups, from the sequence's own context, which the
+// table's width only bounds: equal parts of at least least_part tiles, none for contexts of up to
+// whole_tiles tiles.
+__host__ __device__ inline int prefill_part_tiles(const PrefillArgs& p, int ctx) {
+    const int T = (ctx + p.tile_tokens - 1) >> (p.tile_tokens == 64 ? 6 : 5);
+    if (T <= p.whole_tiles) return T;
+    const int len = (int)(((unsigned long long)(unsigned)(T + p.splits - 1) * p.splits_magic) >> 32);  // ceil(T / splits)
+    return len > p.least_part ? len : p.least_part;
+}
 
 hipError_t launch_attention_prefill(const PrefillArgs& p, hipStream_t stream);
 

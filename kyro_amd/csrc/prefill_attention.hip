@@ -18,10 +18,11 @@
 //     to the end whatever the lengths.
 //   * attn_prefill_combine_kernel: merges the partial states of row groups split into parts.
 // Workgroup w takes kv head w % Hkv of list entry w / Hkv: with 8 kv heads the dispatcher's
-// round-robin over the 8 XCDs keeps every head's K/V in one XCD's L2. Launches whose row groups
-// all fit the chip at once, or have at most 1024 tokens (f32: 256), skip the list: the workgroup
-// works its row group and part out from its index, the host having chosen the parts
-// (prefill_splits in runtime.cpp).
+// round-robin over the 8 XCDs keeps every head's K/V in one XCD's L2. Launches in which no workgroup
+// has more than 1024 tokens (f32: 256) to walk, and those of one sequence that fit the chip at once, skip
+// the list: the workgroup works its row group and part out from its index. The host bounds the parts
+// (prefill_splits in runtime.cpp, from the table's width), the sequence's own context decides them
+// (prefill_part_tiles): a table as wide as the longest context a server allows does not make them long.
 //
 // What bounds it: at head dim 128 a wave's tile of 64 tokens is 32 MFMAs (1024 cycles), about 215
 // vector instructions (about 1000 cycles, the exponentials a quarter of them) and 24 KiB of LDS
@@ -179,9 +180,10 @@ __global__ __launch_bounds__(kPfThreads, prefill_wgs_per_cu(BF16, DR)) void attn
         const int err = sequence_rows(a, e0.x, e0.y, e0.z, e0.w);
         if (err && rest == 0 && kvh == 0 && threadIdx.x == 0) latch_error(a.err, err);
         const int T = row_group_tiles(p, rg, e0.z, e0.w);
-        if (T < 0 || (s > 0 && s * p.chunk >= T)) return;
-        e1 = make_int4(rg * kPrefillRows, s * p.chunk, min(p.chunk, T - s * p.chunk),
-                       T > p.chunk ? (e0.x * a.row_groups + rg) * p.splits + s : -1);
+        const int len = prefill_part_tiles(p, e0.w);
+        if (T < 0 || (s > 0 && s * len >= T)) return;
+        e1 = make_int4(rg * kPrefillRows, s * len, min(len, T - s * len),
+                       T > len ? (e0.x * a.row_groups + rg) * p.splits + s : -1);
     }
     const int b = __builtin_amdgcn_readfirstlane(e0.x);
     const int q0 = __builtin_amdgcn_readfirstlane(e0.y);
@@ -562,10 +564,11 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_combine_kernel(Prefil
             int ctx;
             if (sequence_rows(a, b, e.x, e.y, ctx)) continue;  // the first pass latched it
             const int T = row_group_tiles(p, rg, e.y, ctx);
-            if (T <= p.chunk) continue;  // stored by the first pass, or no rows
+            const int len = prefill_part_tiles(p, ctx);
+            if (T <= len) continue;  // stored by the first pass, or no rows
             e.z = rg * kPrefillRows;
             f.x = y * p.splits;
-            f.y = (T + p.chunk - 1) / p.chunk;
+            f.y = (T + len - 1) / len;
         }
         const int n = e.z + 32 * wave + col;
         if (n >= e.y * a.group) continue;

@@ -163,12 +163,16 @@ struct AttnSetup {
     size_t ws_bytes = 0;     // arena bytes the launch takes
 };
 
-// Parts that each of `items` row groups of at most `most` tiles is split into when the host decides
-// alone: the least of an estimate in tile times (one workgroup on a CU: about 1.1 us in bf16, 4 us in
-// f32). Workgroups beyond one a CU share it; a split costs the second launch, and each part its
-// 64 KiB to park and to merge.
+// Parts that each of `items` row groups is split into when there is no list, at contexts of `most` tiles
+// (those of the table's width): the least of an estimate in tile times (one workgroup on a CU: about
+// 1.1 us in bf16, 4 us in f32). Workgroups beyond one a CU share it; a split costs the second launch
+// (`fixed`), and each part its 64 KiB to park and to merge (`each` of all, `serial` of a row group).
+struct PrefillCost {
+    double fixed, each, serial;
+    explicit PrefillCost(bool bf16) : fixed(bf16 ? 4.0 : 1.0), each(bf16 ? 0.025 : 0.007), serial(bf16 ? 0.05 : 0.02) {}
+};
 int prefill_splits(long long items, long long most, int num_cus, int wgs_per_cu, bool bf16) {
-    const double fixed = bf16 ? 4.0 : 1.0, each = (bf16 ? 0.025 : 0.007), serial = bf16 ? 0.05 : 0.02;
+    const PrefillCost cost(bf16);
     const double share = wgs_per_cu > 2 ? 0.5 : 0.8;
     double best = 1e30;
     int best_s = 1;
@@ -176,7 +180,7 @@ int prefill_splits(long long items, long long most, int num_cus, int wgs_per_cu,
         const long long len = (most + s - 1) / s;
         const long long per_cu = (items * s + num_cus - 1) / num_cus;
         double t = (double)len * (1.0 + share * (double)(per_cu - 1));
-        if (s > 1) t += fixed + each * (double)(items * s) + serial * s;
+        if (s > 1) t += cost.fixed + cost.each * (double)(items * s) + cost.serial * s;
         if (t < best) {
             best = t;
             best_s = s;
@@ -185,9 +189,9 @@ int prefill_splits(long long items, long long most, int num_cus, int wgs_per_cu,
     return best_s;
 }
 
-// Work bounds and workspace of a launch of the many-row kernel (prefill_attention.hip). False where
-// a bound passes what one launch carries.
-bool prefill_setup(int num_cus, int kv_reuse, AttnSetup& s) {
+// Work bounds and workspace of a launch of the many-row kernel (prefill_attention.hip) whose sequences
+// bring at most `rows` rows per kv head in all. False where a bound passes what one launch carries.
+bool prefill_setup(int num_cus, int kv_reuse, long long rows, AttnSetup& s) {
     kyro::AttnArgs& a = s.a;
     kyro::PrefillArgs& f = s.pf;
     f.tile_tokens = kyro::prefill_tile_tokens(a.dtype_bf16, a.D);
@@ -203,21 +207,38 @@ bool prefill_setup(int num_cus, int kv_reuse, AttnSetup& s) {
     const size_t acc_row = (size_t)(a.D + 31) / 32 * 32 * sizeof(float);
     const bool dense = all <= 2 * groups;  // most sequences have about max_q_len rows
     const bool few = all * a.Hkv * 2 <= f.slots;
-    if (dense && (few || most * f.tile_tokens <= (a.dtype_bf16 ? 1024 : 256))) {
-        const int want = few ? prefill_splits(all * a.Hkv, most, num_cus, f.slots / num_cus, a.dtype_bf16) : 1;
-        f.chunk = (int)((most + want - 1) / want);
-        f.chunk = std::max(f.chunk, 1);
-        f.splits = (int)std::max(1LL, (most + f.chunk - 1) / f.chunk);
+    // No list where all row groups are those of one sequence (parts of equal length are even then), or
+    // where no workgroup has more than 1024 tokens (f32: 256) to go, twice that where the sequences bring
+    // about the same rows: several sequences may differ, and a long one kept whole beside short ones
+    // would run on alone (four of up to 8192 tokens with one row beside eight 64-token prompts, 32/8 heads:
+    // 148 us whole, 35 in parts; 16 of up to 2000 beside eight of 128, 8/2 heads: 39 whole, 20 in
+    // parts). Row groups that would be too long so may make twice as many parts as fit the chip, which
+    // takes no more scratch than the list's.
+    f.splits = few ? prefill_splits(all * a.Hkv, most, num_cus, f.slots / num_cus, a.dtype_bf16) : 1;
+    const bool even = 4 * rows >= 3LL * a.B * a.rows_cap;  // about the same number of rows in every sequence
+    const long long limit = (a.dtype_bf16 ? 1024 : 256) / f.tile_tokens * (few && even ? 2 : 1);
+    auto too_long = [&] { return !(few && a.B == 1) && (most + f.splits - 1) / f.splits > limit; };
+    if (few && too_long()) f.splits = (int)std::max(1LL, std::min({64LL, most, 2LL * f.slots / (all * a.Hkv)}));
+    if (dense && !too_long()) {
+        // n parts of T tiles take T / n + n * each + fixed tile times, least at parts of sqrt(T * each) tiles:
+        // a wide table's parts are at least those of 32 tiles, and what splitting would not pay for
+        // stays whole. A context as wide as the table makes the parts counted above.
+        const PrefillCost cost(a.dtype_bf16);
+        const double each = cost.each * (double)(all * a.Hkv) + cost.serial;
+        f.splits_magic = (unsigned)((1ull << 32) / (unsigned)f.splits) + 1u;
+        f.least_part = (int)std::min(std::ceil(std::sqrt(32.0 * each)), (double)((most + f.splits - 1) / f.splits));
+        f.least_part = std::max(f.least_part, 1);
+        f.whole_tiles = f.splits == 1 ? INT32_MAX : (int)std::min(f.least_part + (long long)cost.fixed, most - 1);
         if (all * f.splits * a.Hkv * 256 <= 0xffffffffLL) {
             f.list_cap = (int)(all * f.splits);
             f.part_cap = f.splits > 1 ? (int)(all * f.splits) : 0;
-            const size_t rows = (size_t)f.part_cap * a.Hkv * kyro::kPrefillRows;
-            s.ws_bytes = 2 * align_up(rows * sizeof(float), 256) + align_up(rows * acc_row, 256);
+            const size_t part_rows = (size_t)f.part_cap * a.Hkv * kyro::kPrefillRows;
+            s.ws_bytes = 2 * align_up(part_rows * sizeof(float), 256) + align_up(part_rows * acc_row, 256);
             s.kernel = kyro::ATTN_KERNEL_PREFILL;
             return true;
         }
     }
-    f.splits = f.chunk = 0;
+    f.splits = 0;
     // A part is longer than the share ceil(tiles x Hkv / slots), so the row groups that split make
     // at most 2 x slots / Hkv parts; and each at most ceil(longest / (split_cost + 1)).
     long long parts = 0;
@@ -226,10 +247,10 @@ bool prefill_setup(int num_cus, int kv_reuse, AttnSetup& s) {
     if ((groups + parts) * a.Hkv * 256 > 0xffffffffLL) return false;
     f.list_cap = (int)(groups + parts);
     f.part_cap = (int)parts;
-    const size_t rows = (size_t)parts * a.Hkv * kyro::kPrefillRows;
+    const size_t part_rows = (size_t)parts * a.Hkv * kyro::kPrefillRows;
     s.ws_bytes = 256 + align_up((size_t)f.list_cap * 2 * sizeof(int4), 256) +
-                 align_up((size_t)f.part_cap * 2 * sizeof(int4), 256) + 2 * align_up(rows * sizeof(float), 256) +
-                 align_up(rows * acc_row, 256);
+                 align_up((size_t)f.part_cap * 2 * sizeof(int4), 256) + 2 * align_up(part_rows * sizeof(float), 256) +
+                 align_up(part_rows * acc_row, 256);
     s.kernel = kyro::ATTN_KERNEL_PREFILL;
     return true;
 }
@@ -341,7 +362,7 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
         kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, rows, p->batch_size, p->num_kv_heads, (long long)group * max_q_len)) {
         a.ubs = 16;
         a.sub = a.bs / 16;
-        if (prefill_setup(num_cus, p->kv_reuse, s)) return KYRO_OK;
+        if (prefill_setup(num_cus, p->kv_reuse, rows, s)) return KYRO_OK;
         a.ubs = kernel == kyro::ATTN_KERNEL_MFMA ? 16 : p->block_size;
         a.sub = a.bs / a.ubs;
     }
@@ -605,6 +626,16 @@ int kyro_abi_version(void) { return KYRO_ABI_VERSION; }
 
 int64_t kyro_testing_set_plan_slot_cap(int64_t cap) {
     return g_test_plan_slot_cap.exchange(cap < 0 ? 0 : cap, std::memory_order_relaxed);
+}
+
+int kyro_testing_prefill_part_tiles(const kyro_paged_attention_params* p, int has_q_start_loc, int64_t ctx, int* splits) {
+    return guarded([&]() -> int {
+        AttnSetup s;
+        if (int rc = attention_setup(p, has_q_start_loc != 0, kDefaultCUs, s)) return -rc;
+        if (s.kernel != kyro::ATTN_KERNEL_PREFILL) return -KYRO_EUNSUPPORTED;
+        if (splits) *splits = s.pf.splits;
+        return s.pf.splits ? kyro::prefill_part_tiles(s.pf, (int)ctx) : 0;
+    });
 }
 
 int kyro_ctx_create(int device, kyro_ctx* out) {

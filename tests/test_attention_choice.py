@@ -1,9 +1,12 @@
 """Which kernel, schedule and parts an attention call takes, as the library describes its own choice (host
 only; 256 CUs)."""
+import ctypes
+
 import pytest
 import torch
 
 import kyro_amd
+from kyro_amd import _lib
 from kyro_amd.attention import describe_attention
 
 DTYPES = {"bf16": torch.bfloat16, "f32": torch.float32}
@@ -25,3 +28,50 @@ def test_padding_rows_do_not_choose_the_kernel(H, Hkv, D, batch, max_q, blocks, 
     text = describe(H, Hkv, D, batch, max_q, blocks, dtype, total_q=512)
     assert text == describe(H, Hkv, D, batch, max_q, blocks, dtype)
     assert "attn_mfma" in text, text
+
+
+def part_tiles(H, Hkv, D, batch, max_q, blocks, dtype, ctx, total_q=None):
+    """(tiles of a part, most parts) of a sequence of ctx tokens in the many-row kernel; (0, 0) if listed."""
+    p = _lib.PagedAttentionParams(16, H, D, Hkv, batch, total_q or batch * max_q, blocks, batch * blocks,
+                                  _lib.KYRO_BF16 if dtype == "bf16" else _lib.KYRO_F32, _lib.KYRO_BF16, 1, 0.0, 0, 0, max_q, 0, 0)
+    splits = ctypes.c_int()
+    n = _lib.lib().kyro_testing_prefill_part_tiles(ctypes.byref(p), 1, ctx, ctypes.byref(splits))
+    assert n >= 0
+    return n, splits.value
+
+
+@pytest.mark.parametrize("H,Hkv,D,max_q,dtype", [(32, 8, 128, 64, "bf16"), (16, 1, 128, 128, "bf16"), (16, 1, 192, 24, "bf16"),
+                                                 (32, 8, 64, 64, "f32"), (8, 8, 128, 512, "f32")])
+def test_parts_follow_the_context_not_the_table(H, Hkv, D, max_q, dtype):
+    """One sequence of 4096 tokens in tables of 1 to 64 times that width."""
+    tile = 64 if dtype == "bf16" and D <= 128 else 32
+    T = 4096 // tile
+    tight, most = part_tiles(H, Hkv, D, 1, max_q, 256, dtype, 4096)
+    for width in (512, 2048, 16384):
+        n, splits = part_tiles(H, Hkv, D, 1, max_q, width, dtype, 4096)
+        assert n <= tight and -(-T // n) <= splits
+        assert -(-T // n) <= 2 * -(-T // tight)  # nor more parts to merge than twice those of the tight table
+
+
+@pytest.mark.parametrize("blocks", [64, 300, 4096, 60000])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_parts_cover_every_length(blocks, dtype):
+    tile = 64 if dtype == "bf16" else 32
+    for ctx in [0, 1, 2, tile - 1, tile, tile + 1] + [blocks * 16 * i // 97 for i in range(98)]:
+        n, splits = part_tiles(32, 8, 64, 1, 128, blocks, dtype, ctx)
+        T = -(-ctx // tile)
+        assert (n >= 1 or T == 0) and n * splits >= T
+
+
+def test_sequences_that_may_differ_have_short_parts_or_a_list():
+    """Without a list no part of several sequences may pass 1024 tokens (f32: 256) whatever their lengths, or
+    twice that where they bring about the same rows."""
+    # one row on up to 8192 tokens beside 64-token prompts: listed; on up to 2000 beside 128-token ones: parts
+    assert part_tiles(32, 8, 128, 12, 64, 512, "bf16", 8192, total_q=8 * 64 + 4) == (0, 0)
+    n, splits = part_tiles(8, 2, 128, 24, 128, 125, "bf16", 2000, total_q=16 + 8 * 128)
+    assert splits > 1 and n * 64 <= 1024
+    assert part_tiles(16, 1, 128, 2, 128, 8192, "bf16", 4096) == (0, 0)
+    assert part_tiles(32, 8, 64, 4, 32, 4096, "f32", 4096) == (0, 0)
+    n, splits = part_tiles(32, 8, 128, 2, 64, 256, "bf16", 4096)
+    assert splits > 1 and n * 64 <= 1024
+    assert part_tiles(32, 8, 128, 16, 128, 64, "bf16", 1024)[1] == 1

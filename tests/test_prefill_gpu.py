@@ -120,6 +120,23 @@ def test_many_rows_large_values_after_a_much_larger_score(gpu, dtype, D):
     assert float((out - exact).abs().max()) <= (4 * 2.0 ** -9 if dtype == "bf16" else 1e-4) * float(t["value_cache"].abs().max())
 
 
+@pytest.mark.parametrize("dtype,D", [("bf16", 128), ("bf16", 256), ("f32", 64)])
+@pytest.mark.parametrize("heads,ctx,ql", [((8, 1), [5000], [64]), ((8, 2), [700], [512]), ((8, 1), [64], [64]),
+                                          ((16, 1), [3000, 40, 0, 900], [32, 40, 3, 32]), ((8, 2), [0], [200])])
+def test_many_rows_wide_table(gpu, dtype, D, heads, ctx, ql):
+    """Tables of 32768 tokens, as a server that sizes them for its longest context passes: parts by the
+    context of one sequence, a list for several."""
+    case = wl.make_attention_case(context_lens=ctx, q_lens=ql, num_heads=heads[0], num_kv_heads=heads[1], head_dim=D,
+                                  dtype=dtype, seed=D + len(ctx))
+    table = np.zeros((case.batch, 2048), np.int64)
+    table[:, :case.block_table.shape[1]] = case.block_table
+    case.block_table = table
+    assert _takes_many_rows(case)
+    t = h.attention_tensors(case, gpu)
+    out = _attention(case).forward(*_args(t), q_start_loc=t["q_start_loc"])
+    h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32)
+
+
 def test_many_rows_errors_latch(gpu):
     """A bad block id, a context longer than its table and rows out of order are reported; the
     sequences without a fault are computed as before."""
