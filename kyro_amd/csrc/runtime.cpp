@@ -430,21 +430,30 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     splits = (mb + chunk - 1) / chunk;
     // Where the whole batch's chunks of 8, 16 or 32 slots fit the chip at once, the grid takes them:
     // no workgroup has more to do than one chunk, whatever the lengths, so there is nothing for the
-    // balanced schedule to even out and its plan (about 5 us in every workgroup) is saved. The
-    // splits stay few enough that the combine pass does not cost more: 32, or 16 with several row
-    // groups or wide heads. One sequence of 1000 tokens, 32/8 heads, bf16: 16.3 -> 14.5 us a call
-    // (the host's time for two launches; 16 -> 9 us of kernels), f32 26.0 -> 14.8, head dim 256
-    // 31.8 -> 19.4; 12000 tokens, 8/8 heads: 21.5 -> 15.7 with 24 splits, but 25.8 against 22.5
-    // with 94 at 32/8 heads. Short bf16 contexts that took one launch before (up to 496 tokens) keep
-    // it: 300 tokens 11.9 us, 14.6 in chunks (f32 20.1 and 14.8).
+    // balanced schedule to even out and its plan (about 5 us in every workgroup) is saved. "At once" is
+    // one workgroup a CU of the XCD that the grid deals a unit group's splits and row groups to, not of
+    // the chip: with few unit groups the others idle (16/1 heads, f32, 24 rows on 2000 tokens: 26 us
+    // balanced, 74 in 192 workgroups on one XCD). The splits stay few enough that the combine pass does not
+    // cost more: 32, or 16 with several row groups or wide heads. One sequence of 1000 tokens, 32/8 heads,
+    // bf16: 16.3 -> 14.5 us a call (the host's time for two launches; 16 -> 9 us of kernels), f32 26.0 ->
+    // 14.8, head dim 256 31.8 -> 19.4; 12000 tokens, 8/8 heads: 21.5 -> 15.7 with 24 splits, but 25.8 against
+    // 22.5 with 94 at 32/8 heads. Contexts that one launch takes whole keep it in bf16 up to head dim 128
+    // (up to 496 tokens: 300 tokens 11.9 us, 14.6 in chunks). f32 and wider heads are split where the
+    // second launch pays: from three chunks on, and where four waves share a head from 20 slots on (one
+    // sequence, head dim 160: 256 tokens 9.3 us whole, 12.0 in two chunks, 4/1 heads; 400 tokens in four
+    // 0.72 to 0.83 of whole); f32 head pairs also in two chunks of 8 (144 to 256 tokens, 0.86 of whole).
     bool short_chunks = false;
     if ((forms & FORM_SHORT_CHUNKS) && kernel == kyro::ATTN_KERNEL_MFMA && p->num_splits == 0 &&
         p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (splits > 1 || p->dtype == KYRO_F32 || p->head_dim > 128)) {
         const long long groups = (long long)a.ugroups * a.row_groups;
+        const long long per_xcd = (long long)(a.ugroups_padded / 8) * a.row_groups;  // map_workgroup
         const bool narrow = a.row_groups == 1 && p->head_dim <= 128;
+        const bool split_anyway = splits > 1 || mb > 256;  // the grid or the balanced schedule would
         for (int c : {8, 16, 32}) {
             const int n = (mb + c - 1) / c;
-            if (n < 2 || n > (narrow ? 32 : 16) || groups * n > num_cus) continue;
+            if (n < 2 || n > (narrow ? 32 : 16) || per_xcd * n > num_cus / 8) continue;
+            if (!split_anyway && !(n >= 3 && (a.hpw == 2 || mb >= 20)) && !(p->dtype == KYRO_F32 && a.hpw == 2 && c == 8))
+                continue;
             // 32 slots only where the balanced schedule's own chunk (5/4 of a CU's share) would be
             // about as long: at few groups its shorter ones win (12000 tokens, 32/8 heads, f32: 33.0
             // against 40.0 us).

@@ -75,3 +75,24 @@ def test_sequences_that_may_differ_have_short_parts_or_a_list():
     n, splits = part_tiles(32, 8, 128, 2, 64, 256, "bf16", 4096)
     assert splits > 1 and n * 64 <= 1024
     assert part_tiles(32, 8, 128, 16, 128, 64, "bf16", 1024)[1] == 1
+
+
+@pytest.mark.parametrize("H,Hkv,D,batch,max_q,blocks,dtype,want", [
+    # the splits and row groups of a unit group share an XCD: few unit groups do not fill the chip
+    (16, 1, 128, 1, 24, 125, "f32", "schedule balanced"),
+    (16, 1, 192, 1, 8, 256, "bf16", "schedule balanced"),
+    (8, 2, 224, 2, 32, 256, "bf16", "schedule balanced"),
+    (28, 4, 128, 1, 24, 125, "f32", "schedule balanced"),
+    (16, 1, 96, 1, 1, 256, "bf16", "schedule grid, row groups 1, splits 32,"),
+    # one launch takes these whole; two chunks cost more than they save
+    (16, 1, 160, 1, 1, 16, "bf16", "schedule grid, row groups 1, splits 1,"),
+    (28, 4, 160, 32, 4, 19, "bf16", "schedule grid, row groups 2, splits 1,"),
+    (32, 32, 64, 4, 1, 19, "f32", "schedule grid, row groups 1, splits 1,"),
+    (4, 4, 64, 1, 8, 16, "f32", "schedule grid, row groups 1, splits 1,"),
+    (32, 8, 160, 1, 1, 19, "bf16", "schedule grid, row groups 1, splits 3,"),
+    (32, 8, 128, 1, 1, 9, "f32", "schedule grid, row groups 1, splits 2,"),
+    (4, 4, 160, 1, 1, 25, "bf16", "schedule grid, row groups 1, splits 4,"),
+])
+def test_short_chunks_where_they_fit_and_pay(H, Hkv, D, batch, max_q, blocks, dtype, want):
+    text = describe(H, Hkv, D, batch, max_q, blocks, dtype)
+    assert want in text, text
