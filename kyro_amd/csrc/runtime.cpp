@@ -255,6 +255,20 @@ bool prefill_setup(int num_cus, int kv_reuse, long long rows, AttnSetup& s) {
     return true;
 }
 
+// Whether the kernels that stream K/V per wave take short contexts (`slots` of 16 tokens) faster than the
+// many-row kernel: where their workgroups are one round, at most one a CU of the XCDs the grid deals them
+// to, and the contexts too short to share. f32 up to 128 tokens (head dim 128, four 128-token prompts,
+// 28/4 heads: 20.1 against 25.2 us; at 300 tokens 0.6 of the time there) or, at head dim 128 with four waves
+// on a head, 304 (8/1 heads, 256 tokens: 19.2 against 26.2); bf16 above head dim 128 with four waves on a
+// head up to 496 (8/8 heads, head dim 256, 256 tokens: 14.4 against 20.9), or 512 with every CU taken
+// (below that the splits need the balanced schedule: 30.4 against 17.4).
+bool one_round_wins(const AttnSetup& s, long long slots, int num_cus) {
+    const kyro::AttnArgs& a = s.a;
+    if ((long long)(a.ugroups_padded / 8) * a.row_groups > num_cus / 8) return false;
+    if (!a.dtype_bf16) return slots <= (a.D == 128 && a.hpw == 1 ? 19 : 8);
+    return a.D > 128 && a.hpw == 1 && slots <= ((long long)a.ugroups * a.row_groups >= num_cus ? 32 : 31);
+}
+
 // Forms of a launch that automatic choice may take beside the grid and the balanced schedule.
 enum AttnForms : int {
     FORM_MANY_ROWS = 1,     // the many-row kernel
@@ -354,18 +368,6 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
     const double scale = p->scale > 0 ? (double)p->scale : 1.0 / std::sqrt((double)p->head_dim);
     a.scale_log2 = (float)(scale * 1.4426950408889634);
     a.units = p->batch_size * p->num_kv_heads;
-    // Rows the sequences can bring: padding rows of q belong to none.
-    const long long rows = std::min<long long>(p->total_q, (long long)p->batch_size * max_q_len) * group;
-    if ((forms & FORM_MANY_ROWS) && mfma_blocks && kyro::prefill_head_dim(p->head_dim, p->dtype == KYRO_BF16) &&
-        (p->path == KYRO_ATTN_AUTO || (p->path == KYRO_ATTN_MFMA && mfma_ok)) && p->num_splits <= 0 &&
-        p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (long long)p->max_blocks_per_seq * p->block_size < (1ll << 30) &&
-        kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, rows, p->batch_size, p->num_kv_heads, (long long)group * max_q_len)) {
-        a.ubs = 16;
-        a.sub = a.bs / 16;
-        if (prefill_setup(num_cus, p->kv_reuse, rows, s)) return KYRO_OK;
-        a.ubs = kernel == kyro::ATTN_KERNEL_MFMA ? 16 : p->block_size;
-        a.sub = a.bs / a.ubs;
-    }
     // Row groups: a unit's group * max_q_len query rows are spread over workgroups of 8
     // (vector) or 16 / 32 / 64 / 80 (MFMA) rows that stream the same K/V. The five-tile choice
     // reads the average rows per kv head from total_q (an upper bound when q has padding rows).
@@ -404,6 +406,22 @@ int attention_setup(const kyro_paged_attention_params* p, bool have_q_start, int
         return fail(KYRO_EUNSUPPORTED, "paged_attention: max_blocks_per_seq %d x block_size %d tokens is too long",
                     p->max_blocks_per_seq, p->block_size);
     const int mb = (int)mb_slots;
+    // Rows the sequences can bring: padding rows of q belong to none.
+    const long long rows = std::min<long long>(p->total_q, (long long)p->batch_size * max_q_len) * group;
+    if ((forms & FORM_MANY_ROWS) && mfma_blocks && kyro::prefill_head_dim(p->head_dim, p->dtype == KYRO_BF16) &&
+        (p->path == KYRO_ATTN_AUTO || (p->path == KYRO_ATTN_MFMA && mfma_ok)) && p->num_splits <= 0 &&
+        p->schedule == KYRO_ATTN_SCHEDULE_AUTO && (long long)p->max_blocks_per_seq * p->block_size < (1ll << 30) &&
+        kyro::prefill_rows(p->dtype == KYRO_BF16, p->head_dim, rows, p->batch_size, p->num_kv_heads,
+                           (long long)group * max_q_len) &&
+        !one_round_wins(s, mb_slots, num_cus)) {
+        AttnSetup many = s;
+        many.a.ubs = 16;
+        many.a.sub = a.bs / 16;
+        if (prefill_setup(num_cus, p->kv_reuse, rows, many)) {
+            s = many;
+            return KYRO_OK;
+        }
+    }
     int splits = p->num_splits;
     if (splits <= 0) {
         // At most ~256 blocks (4096 tokens) per workgroup so a long context does not leave

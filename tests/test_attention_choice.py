@@ -96,3 +96,23 @@ def test_sequences_that_may_differ_have_short_parts_or_a_list():
 def test_short_chunks_where_they_fit_and_pay(H, Hkv, D, batch, max_q, blocks, dtype, want):
     text = describe(H, Hkv, D, batch, max_q, blocks, dtype)
     assert want in text, text
+
+
+@pytest.mark.parametrize("H,Hkv,D,batch,max_q,blocks,dtype,many", [
+    # short contexts in one round of workgroups stay with the kernels that stream K/V per wave
+    (8, 8, 256, 2, 256, 16, "bf16", False),
+    (8, 8, 224, 1, 512, 32, "bf16", False),
+    (4, 4, 192, 2, 300, 32, "bf16", True),    # fewer workgroups than CUs: split, so scheduled on the device
+    (8, 8, 256, 4, 256, 16, "bf16", True),    # two rounds
+    (32, 8, 256, 1, 64, 16, "bf16", True),    # two waves a head
+    (8, 8, 128, 2, 256, 16, "bf16", True),
+    (28, 4, 128, 4, 128, 8, "f32", False),
+    (28, 4, 128, 4, 128, 19, "f32", True),
+    (8, 1, 128, 1, 256, 19, "f32", True),     # one kv head: its row groups queue on one XCD
+    (8, 1, 128, 8, 64, 19, "f32", False),
+    (8, 2, 112, 1, 64, 4, "f32", False),
+    (8, 2, 112, 1, 64, 9, "f32", True),
+])
+def test_one_round_of_short_contexts_keeps_its_kernel(H, Hkv, D, batch, max_q, blocks, dtype, many):
+    text = describe(H, Hkv, D, batch, max_q, blocks, dtype)
+    assert ("attn_prefill_kernel" in text) == many, text
