@@ -213,12 +213,14 @@ bool prefill_setup(int num_cus, int kv_reuse, long long rows, AttnSetup& s) {
     // would run on alone (four of up to 8192 tokens with one row beside eight 64-token prompts, 32/8 heads:
     // 148 us whole, 35 in parts; 16 of up to 2000 beside eight of 128, 8/2 heads: 39 whole, 20 in
     // parts). Row groups that would be too long so may make twice as many parts as fit the chip, which
-    // takes no more scratch than the list's.
+    // takes no more scratch than the list's; of about the same rows, as few as keep the limit (64/8 heads,
+    // 32 sequences of 4096 tokens with 8 rows: 94 us whole, 97 in two parts, 109 in four).
     f.splits = few ? prefill_splits(all * a.Hkv, most, num_cus, f.slots / num_cus, a.dtype_bf16) : 1;
     const bool even = 4 * rows >= 3LL * a.B * a.rows_cap;  // about the same number of rows in every sequence
     const long long limit = (a.dtype_bf16 ? 1024 : 256) / f.tile_tokens * (few && even ? 2 : 1);
     auto too_long = [&] { return !(few && a.B == 1) && (most + f.splits - 1) / f.splits > limit; };
-    if (few && too_long()) f.splits = (int)std::max(1LL, std::min({64LL, most, 2LL * f.slots / (all * a.Hkv)}));
+    if (few && too_long())
+        f.splits = (int)std::max(1LL, std::min({64LL, even ? (most + limit - 1) / limit : most, 2LL * f.slots / (all * a.Hkv)}));
     if (dense && !too_long()) {
         // n parts of T tiles take T / n + n * each + fixed tile times, least at parts of sqrt(T * each) tiles:
         // a wide table's parts are at least those of 32 tiles, and what splitting would not pay for

@@ -116,3 +116,7 @@ def test_short_chunks_where_they_fit_and_pay(H, Hkv, D, batch, max_q, blocks, dt
 def test_one_round_of_short_contexts_keeps_its_kernel(H, Hkv, D, batch, max_q, blocks, dtype, many):
     text = describe(H, Hkv, D, batch, max_q, blocks, dtype)
     assert ("attn_prefill_kernel" in text) == many, text
+
+
+def test_even_sequences_make_no_more_parts_than_they_need():
+    assert part_tiles(64, 8, 128, 32, 8, 256, "bf16", 4096) == (32, 2)
