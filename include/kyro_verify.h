@@ -212,8 +212,9 @@ int kyro_paged_attention_workspace(kyro_ctx ctx, const kyro_paged_attention_para
                                    int has_q_start_loc, size_t* bytes);
 
 /* What a kyro_paged_attention_mq call with these params launches (kernel instance, schedule,
- * splits, workgroups), as text for logs and benchmarks. Host only, like the workspace query; ctx
- * may be NULL (a 256-CU device). buf gets at most len bytes (terminated), *needed (may be NULL)
+ * splits, workgroups), as text for logs and benchmarks, for caches that start on 16-byte boundaries
+ * (others do not take the many-row kernel) and an arena that may grow. Host only, like the workspace
+ * query; ctx may be NULL (a 256-CU device). buf gets at most len bytes (terminated), *needed (may be NULL)
  * the full length with its terminator. No counterpart in the reference. */
 int kyro_paged_attention_describe(kyro_ctx ctx, const kyro_paged_attention_params* params, int has_q_start_loc,
                                   char* buf, size_t len, size_t* needed);

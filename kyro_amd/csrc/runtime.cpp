@@ -927,12 +927,14 @@ int kyro_paged_attention_describe(kyro_ctx ctx, const kyro_paged_attention_param
         const kyro::AttnArgs& a = s.a;
         char t[512];
         if (s.kernel == kyro::ATTN_KERNEL_PREFILL) {
+            char work[128];
+            if (s.pf.splits) std::snprintf(work, sizeof work, "parts per row group up to %d", s.pf.splits);
+            else std::snprintf(work, sizeof work, "listed by attn_prefill_plan_kernel, split parts up to %d", s.pf.part_cap);
             std::snprintf(t, sizeof t,
                           "attn_prefill_kernel<%s, head_dim %d> %d rows per workgroup, tiles of %d tokens, row groups %d, "
-                          "parts up to %d, workgroups up to %lld (+ attn_prefill_plan_kernel%s)",
-                          a.dtype_bf16 ? "bf16" : "f32", a.D, kyro::kPrefillRows, s.pf.tile_tokens, a.row_groups,
-                          s.pf.part_cap, (long long)s.pf.list_cap * a.Hkv,
-                          s.pf.part_cap > 0 ? ", attn_prefill_combine_kernel" : "");
+                          "%s, workgroups up to %lld%s (caches on 16-byte boundaries)",
+                          a.dtype_bf16 ? "bf16" : "f32", a.D, kyro::kPrefillRows, s.pf.tile_tokens, a.row_groups, work,
+                          (long long)s.pf.list_cap * a.Hkv, s.pf.part_cap > 0 ? " + attn_prefill_combine_kernel" : "");
         } else if (s.kernel == kyro::ATTN_KERNEL_MFMA) {
             const int rpg = a.rows_per_group;
             const char* pol = a.stream_kv == kyro::kKvPerUnit ? "per-unit" : a.stream_kv ? "stream" : "cached";

@@ -120,3 +120,15 @@ def test_one_round_of_short_contexts_keeps_its_kernel(H, Hkv, D, batch, max_q, b
 
 def test_even_sequences_make_no_more_parts_than_they_need():
     assert part_tiles(64, 8, 128, 32, 8, 256, "bf16", 4096) == (32, 2)
+
+
+def test_describe_names_what_the_many_row_kernel_launches():
+    """The plan kernel only where the work is listed, the merge only where there may be parts."""
+    listed = describe(32, 8, 64, 6, 512, 500)
+    assert "listed by attn_prefill_plan_kernel" in listed and "+ attn_prefill_combine_kernel" in listed
+    parts = describe(32, 8, 128, 1, 64, 256)
+    assert "attn_prefill_plan_kernel" not in parts and "parts per row group up to 13" in parts
+    assert "+ attn_prefill_combine_kernel" in parts
+    whole = describe(32, 8, 128, 16, 128, 64)
+    assert "parts per row group up to 1," in whole
+    assert "plan" not in whole and "combine" not in whole and "16-byte" in whole
