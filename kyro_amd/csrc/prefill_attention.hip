@@ -637,9 +637,7 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_combine_kernel(Prefil
 template <bool BF16, int DR>
 void launch_prefill_dim(const PrefillArgs& p, hipStream_t stream) {
     const dim3 grid((unsigned)((long long)p.list_cap * p.a.Hkv));
-    // The streaming form is built where prefill_rows sends single row groups.
-    constexpr int kOnce = BF16 && DR == 128 ? kLoadStream : kLoadCached;
-    if (p.a.stream_kv) attn_prefill_kernel<BF16, DR, kOnce><<<grid, kPfThreads, 0, stream>>>(p);
+    if (p.a.stream_kv) attn_prefill_kernel<BF16, DR, kLoadStream><<<grid, kPfThreads, 0, stream>>>(p);
     else attn_prefill_kernel<BF16, DR, kLoadCached><<<grid, kPfThreads, 0, stream>>>(p);
     if (p.part_cap > 0) {
         constexpr long long kMaxGrid = 2048;

@@ -199,7 +199,9 @@ bool prefill_setup(int num_cus, int kv_reuse, long long rows, AttnSetup& s) {
     f.split_cost = a.dtype_bf16 ? 6 : 2;
     a.rows_per_group = kyro::kPrefillRows;
     a.row_groups = (a.rows_cap + kyro::kPrefillRows - 1) / kyro::kPrefillRows;
-    a.stream_kv = kv_reuse == KYRO_KV_REUSE_STREAM || (kv_reuse == KYRO_KV_REUSE_AUTO && a.row_groups == 1);
+    // Automatic streaming where prefill_rows sends single row groups that read each slab once.
+    a.stream_kv = kv_reuse == KYRO_KV_REUSE_STREAM ||
+                  (kv_reuse == KYRO_KV_REUSE_AUTO && a.row_groups == 1 && a.dtype_bf16 && a.D == 128);
     const long long all = (long long)a.B * a.row_groups;
     const long long groups = std::min(all, (long long)a.total_q * a.group / kyro::kPrefillRows + a.B);
     if (all > INT32_MAX) return false;
@@ -931,9 +933,9 @@ int kyro_paged_attention_describe(kyro_ctx ctx, const kyro_paged_attention_param
             if (s.pf.splits) std::snprintf(work, sizeof work, "parts per row group up to %d", s.pf.splits);
             else std::snprintf(work, sizeof work, "listed by attn_prefill_plan_kernel, split parts up to %d", s.pf.part_cap);
             std::snprintf(t, sizeof t,
-                          "attn_prefill_kernel<%s, head_dim %d> %d rows per workgroup, tiles of %d tokens, row groups %d, "
+                          "attn_prefill_kernel<%s, head_dim %d, K/V loads %s> %d rows per workgroup, tiles of %d tokens, row groups %d, "
                           "%s, workgroups up to %lld%s (caches on 16-byte boundaries)",
-                          a.dtype_bf16 ? "bf16" : "f32", a.D, kyro::kPrefillRows, s.pf.tile_tokens, a.row_groups, work,
+                          a.dtype_bf16 ? "bf16" : "f32", a.D, a.stream_kv ? "stream" : "cached", kyro::kPrefillRows, s.pf.tile_tokens, a.row_groups, work,
                           (long long)s.pf.list_cap * a.Hkv, s.pf.part_cap > 0 ? " + attn_prefill_combine_kernel" : "");
         } else if (s.kernel == kyro::ATTN_KERNEL_MFMA) {
             const int rpg = a.rows_per_group;

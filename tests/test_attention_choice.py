@@ -132,3 +132,11 @@ def test_describe_names_what_the_many_row_kernel_launches():
     whole = describe(32, 8, 128, 16, 128, 64)
     assert "parts per row group up to 1," in whole
     assert "plan" not in whole and "combine" not in whole and "16-byte" in whole
+
+
+@pytest.mark.parametrize("D,dtype", [(64, "bf16"), (128, "bf16"), (256, "bf16"), (64, "f32"), (128, "f32")])
+def test_many_row_kernel_follows_the_reuse_hint(D, dtype):
+    for reuse, want in (("stream", "stream"), ("shared", "cached"), ("auto", "cached")):
+        assert f"attn_prefill_kernel<{dtype}, head_dim {D}, K/V loads {want}>" in describe(32, 8, D, 2, 512, 64, dtype,
+                                                                                       kv_reuse=reuse)
+    assert "K/V loads stream" in describe(64, 8, 128, 64, 9, 256)  # each slab read once

@@ -137,6 +137,15 @@ def test_many_rows_wide_table(gpu, dtype, D, heads, ctx, ql):
     h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32)
 
 
+@pytest.mark.parametrize("dtype,D", DIMS, ids=lambda x: str(x))
+def test_many_rows_reuse_hint_never_changes_the_result(gpu, dtype, D):
+    case = _case("ragged", dtype, D, seed=13)
+    assert _takes_many_rows(case)
+    t = h.attention_tensors(case, gpu)
+    outs = [_attention(case).forward(*_args(t), q_start_loc=t["q_start_loc"], kv_reuse=r) for r in ("auto", "shared", "stream")]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 def test_many_rows_errors_latch(gpu):
     """A bad block id, a context longer than its table and rows out of order are reported; the
     sequences without a fault are computed as before."""
