@@ -133,7 +133,7 @@ class PagedAttention:
         if out_dtype not in _DTYPES:
             raise TypeError(f"out_dtype must be float32 or bfloat16, got {out_dtype}")
         if out is None:
-            out = (torch.empty_like(query) if out_dtype == dtype and type(query) is torch.Tensor
+            out = (torch.empty_like(query, memory_format=torch.contiguous_format) if out_dtype == dtype and type(query) is torch.Tensor
                    else torch.empty((total_q, h, d), dtype=out_dtype, device=dev))
         else:
             _require(out, "out", dtype=out_dtype, ndim=3, device=dev)

@@ -708,3 +708,14 @@ def test_mha_b2_matches_golden_fixture(gpu, path):
         q_start_loc=t["q_start_loc"], path=path)
     err = (out.cpu().numpy() - z["expected"]).__abs__().max()
     assert err <= h.ATOL_BF16, err
+
+
+def test_output_of_one_row_has_plain_strides(gpu):
+    """A contiguous query of one row may carry any stride in that dimension; the output's are its own."""
+    case = wl.make_attention_case(context_lens=[9], q_lens=[1], num_heads=8, num_kv_heads=2, dtype="bf16", seed=31)
+    t = h.attention_tensors(case, gpu)
+    q = t["query"].as_strided((1, 8, 128), (7, 128, 1))
+    assert q.is_contiguous()
+    out = make_attention(16, 8, 128, 2).forward(q, t["key_cache"], t["value_cache"], t["block_table"], t["context_lens"],
+                                                out_dtype=torch.bfloat16)
+    assert out.stride() == (8 * 128, 128, 1)
