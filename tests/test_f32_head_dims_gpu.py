@@ -39,7 +39,7 @@ def test_f32_head_dims_parity(gpu, name, D):
                 t[x][int(case.block_table[b, n // block]), :, n % block:, :] = float("nan")
     out = attn.forward(t["query"], t["key_cache"], t["value_cache"], t["block_table"], t["context_lens"],
                        q_start_loc=t["q_start_loc"], num_splits=splits)
-    h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_F32)
+    h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_F32_SUMS)
 
 
 def test_f32_head_dims_stay_refused_by_name(gpu):

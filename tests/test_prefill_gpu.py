@@ -52,16 +52,15 @@ def _takes_many_rows(case):
         max_blocks_per_seq=case.block_table.shape[1], num_blocks=case.key_cache.shape[0], dtype=dtype)
 
 
-@pytest.mark.parametrize("dtype,D", DIMS, ids=lambda x: str(x))
-@pytest.mark.parametrize("name", sorted(EDGES))
+# 72 rows per kv head take this kernel in bf16 at head dim 128 alone.
+@pytest.mark.parametrize("name,dtype,D", [(name, dtype, D) for name in sorted(EDGES) for dtype, D in DIMS
+                                          if name != "verify72" or (dtype, D) == ("bf16", 128)], ids=lambda x: str(x))
 def test_many_rows_parity(gpu, name, dtype, D):
-    if name == "verify72" and (dtype, D) != ("bf16", 128):
-        pytest.skip("these rows take another kernel")
     case = _case(name, dtype, D, block=32 if D % 96 == 0 else 16)
     t = h.attention_tensors(case, gpu)
     exp = h.oracle_attention(case)
     out = _attention(case).forward(*_args(t), q_start_loc=t["q_start_loc"])
-    h.assert_attention_close(out, case, exp, h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32)
+    h.assert_attention_close(out, case, exp, h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32_SUMS)
 
 
 def test_the_edges_reach_the_many_row_kernel():
@@ -134,7 +133,7 @@ def test_many_rows_wide_table(gpu, dtype, D, heads, ctx, ql):
     assert _takes_many_rows(case)
     t = h.attention_tensors(case, gpu)
     out = _attention(case).forward(*_args(t), q_start_loc=t["q_start_loc"])
-    h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32)
+    h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32_SUMS)
 
 
 @pytest.mark.parametrize("dtype,D", DIMS, ids=lambda x: str(x))
@@ -190,12 +189,19 @@ def test_many_rows_replay_from_a_graph(gpu, name):
 
 
 def test_many_rows_misaligned_cache_takes_another_kernel(gpu):
-    """Caches that start 2 bytes off a 16-byte boundary run, on the general kernels."""
-    case = _case("gqa7", "bf16", 128, seed=11)
+    """Caches that start 8 bytes off a 16-byte boundary run on the kernels that stream K/V per wave: bit for
+    bit what the grid schedule by name gives, and not what the many-row kernel gives."""
+    case = _case("edges", "bf16", 128, seed=11)
+    assert _takes_many_rows(case)
     t = h.attention_tensors(case, gpu)
+    kw = dict(q_start_loc=t["q_start_loc"])
+    many = _attention(case).forward(*_args(t), **kw)
+    grid = _attention(case).forward(*_args(t), schedule="grid", **kw)
     for x in ("key_cache", "value_cache"):
         flat = torch.zeros(t[x].numel() + 8, dtype=torch.bfloat16, device=gpu)
         flat[4:4 + t[x].numel()] = t[x].flatten()
         t[x] = flat[4:4 + t[x].numel()].view(t[x].shape)
-    out = _attention(case).forward(*_args(t), q_start_loc=t["q_start_loc"])
+        assert t[x].data_ptr() % 16 == 8
+    out = _attention(case).forward(*_args(t), **kw)
     h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16)
+    assert torch.equal(out, grid) and not torch.equal(out, many)

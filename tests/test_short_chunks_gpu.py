@@ -50,7 +50,7 @@ def test_short_chunks_parity(gpu, dtype, H, Hkv, D, ctx, ql):
     t = h.attention_tensors(case, gpu)
     out = attn.forward(t["query"], t["key_cache"], t["value_cache"], t["block_table"], t["context_lens"],
                        q_start_loc=t["q_start_loc"])
-    h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32)
+    h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32_SUMS)
 
 
 @pytest.mark.gpu
@@ -83,6 +83,6 @@ def test_capture_without_a_reserve_takes_a_form_without_scratch(gpu, dtype, H, H
         out.zero_()
         g.replay()
         torch.cuda.synchronize()
-        h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32)
+        h.assert_attention_close(out, case, h.oracle_attention(case), h.ATOL_BF16 if dtype == "bf16" else h.ATOL_F32_SUMS)
     del g
     context.sync()
