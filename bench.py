@@ -521,8 +521,8 @@ def shape_sweep_workload(kind, warmup, steps):
     or other block sizes ("block-sizes": 8, 16, 32, 64 at head_dim 128; AUTO takes the MFMA
     kernel at every multiple of 16, the vector kernel at 8), AUTO and the vector kernel, each on
     its algorithmic bytes; or ("row-tiles") GQA 64/8 at head_dim 128 with 1, 2, 4, 8 and 9 query
-    rows per sequence (8 to 72 rows per kv head: the one-, two-, four- and five-tile MFMA
-    kernels), AUTO only."""
+    rows per sequence (8 to 72 rows per kv head: the one- and two-tile MFMA kernels, and from 64
+    rows on the many-row kernel), AUTO only."""
     import torch
 
     import kyro_amd

@@ -131,8 +131,9 @@ typedef enum kyro_attn_path {
  *   AUTO:   streaming when each slab is read by one workgroup, i.e. a kv head's query rows
  *           (GQA group x max_q_len) fit one row group (16, 32, 64 or 80 rows for bf16
  *           caches); cached otherwise. With 64- and 80-row groups the choice is made per
- *           sequence: those whose rows fit one group stream. Right when no two sequences of the
- *           batch share a block.
+ *           sequence: those whose rows fit one group stream. The kernel for many query rows
+ *           streams in bf16 at head_dim 128 where a kv head's rows fit one group of 128. Right
+ *           when no two sequences of the batch share a block.
  *   SHARED: cached loads; for tables that share blocks between sequences (prefix caching;
  *           kyro_bm_write_tables reports it).
  *   STREAM: streaming loads regardless. */
@@ -144,8 +145,12 @@ typedef enum kyro_kv_reuse {
 
 /* How the MFMA kernel spreads work over the chip. Results do not depend on it beyond float
  * rounding of split merges.
- *   AUTO:     BALANCED when num_splits is 0, the batch has at most 1024 sequences and either
- *             max_blocks_per_seq > 256 or GRID would split contexts; GRID otherwise.
+ *   AUTO:     with num_splits 0, calls with many query rows per kv head use neither: their kernel
+ *             hands its work out by the context lengths. Otherwise GRID in chunks of 128, 256 or 512
+ *             tokens where those of the whole batch, as counted from max_blocks_per_seq, run at once
+ *             (small batches on tables of up to some thousand tokens); else BALANCED when
+ *             num_splits is 0, the batch has at most 1024 sequences and either max_blocks_per_seq >
+ *             256 (slots of 16 tokens) or GRID would split contexts; GRID otherwise.
  *   GRID:     one workgroup per (sequence, kv head pair, context split, row group), with
  *             num_splits splits of max_blocks_per_seq (0: chosen from the shapes alone).
  *   BALANCED: a persistent grid of one workgroup per CU reads the context lengths on the
@@ -203,8 +208,9 @@ int kyro_paged_attention_mq(kyro_ctx ctx, const kyro_paged_attention_params* par
                             const int64_t* block_table, const int64_t* context_lens,
                             void* out);
 
-/* Scratch bytes a kyro_paged_attention_mq call with these params takes from the context's arena
- * (has_q_start_loc: whether the call passes q_start_loc). Host only, no device work; ctx may be
+/* Scratch bytes a kyro_paged_attention_mq call with these params takes at most from the context's
+ * arena (has_q_start_loc: whether the call passes q_start_loc), wherever its caches start: the larger
+ * need where caches off a 16-byte boundary take another kernel. Host only, no device work; ctx may be
  * NULL, which sizes for a 256-CU device. A caller that captures calls into a HIP graph passes the
  * largest of these to kyro_ctx_reserve first. No counterpart in the reference (candle allocates
  * per op). */

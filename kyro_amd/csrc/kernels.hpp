@@ -156,7 +156,8 @@ constexpr int kVectorRowsPerGroup = 8;
 // Five tiles (kMfmaWideRows) where they take fewer row groups than four and the batch's
 // average unit (total_rows / seqs rows per kv head) fills more than half of what the last
 // 64-row group would hold: GQA 64/8 with 8 drafts on every sequence (72 rows a unit) then
-// streams each unit's K/V once instead of twice (B 64, ctx 4096: 331 -> 235 us). The five-tile
+// streams each unit's K/V once instead of twice (B 64, ctx 4096: 331 -> 235 us; batches that large
+// now take the many-row kernel, those of under 8192 rows over the kv heads come here). The five-tile
 // kernel copies about 1.7x as many values through AGPRs per block pair as the four-tile one (both
 // hold more than the 256 VGPRs a wave can address), so a batch with few such units keeps four
 // (mixed GQA 64/8, 0-8 drafts: 385 us with four, 396 with five).
@@ -176,7 +177,8 @@ inline int mfma_rows_per_group(int rows, bool bf16, int D, long long total_rows,
 }
 
 // Head dims the bf16 MFMA kernel is built for: every multiple of 32 from 64 to 256, and 80 and 112
-// in the operand layouts of 96 and 128; f32 caches take it at 128 only.
+// in the operand layouts of 96 and 128. With f32 caches 128 is the head dim that may be asked for by name
+// (mfma_f32_auto_dim has the others).
 __host__ __device__ inline bool mfma_head_dim(int D, bool bf16) {
     return D == 128 || (bf16 && ((D % 32 == 0 && D >= 64 && D <= 256) || D == 80 || D == 112));
 }

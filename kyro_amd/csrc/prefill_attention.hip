@@ -28,11 +28,13 @@
 // vector instructions (about 1000 cycles, the exponentials a quarter of them) and 24 KiB of LDS
 // reads (192 cycles of the CU's LDS unit, times 8 waves a CU), of which two waves a SIMD overlap a
 // part: matrix cores busy 39%, vector units 49% of the time. Without the softmax the same launch
-// takes 148 of 179 us, without the copies 159. At head dim 64 the vector work sets the pace.
-// Measured (us, before -> here): four 2048-token prompts, 32/8 heads, head dim 128: 797 -> 164;
-// 300-512 new tokens on contexts of 700-8000, 32/8 heads, head dim 64: 342 -> 135; one 64-token
-// chunk on a context of 4096, 32/8 heads: 32.4 -> 25.5; f32 four 1024-token chunks, head dim 64:
-// 692 -> 104.
+// takes 83% of its time, without the copies 89%. At head dim 64 the vector work sets the pace.
+// Measured (us a call with plan and merge, the kernels that stream K/V per wave -> here, on one box):
+// four 2048-token prompts, 32/8 heads, head dim 128: 796 -> 183; 300-512 new tokens on contexts of
+// 700-8000, 32/8 heads, head dim 64: 341 -> 148; one 64-token chunk on a context of 4096, 32/8 heads:
+// 31.7 -> 24.6; four 1024-token prompts, 32/8 heads, head dim 64, f32: 1890 -> 207 (the vector kernel).
+// Registers that the workgroups wanted on a CU do not allow (prefill_wgs_per_cu) are spilled, bytes a
+// lane: bf16 at head dim 64 8, 96 12, 256 64; f32 at 128 8.
 #ifndef KYRO_PREFILL_UNIT
 #define KYRO_PREFILL_UNIT 0
 #endif
