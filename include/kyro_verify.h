@@ -231,8 +231,9 @@ int kyro_paged_attention_describe(kyro_ctx ctx, const kyro_paged_attention_param
  * reference. num_cus 0 means 256; chunk_quarters 0 means the library's chunk length (a sequence
  * longer than the per-workgroup share L of the work splits into chunks of about
  * L x chunk_quarters / 4 blocks, 5L/4 by default; other values model other chunk lengths, the
- * slot bound included). Fails with KYRO_EINVAL when the params
- * would run on the grid schedule. out_splits [B] (may be NULL): splits per sequence (0 for a
+ * slot bound included). Under automatic schedule it answers as if neither short chunks nor the kernel
+ * for many query rows took the call, and fails with KYRO_EINVAL when the params
+ * would run on the grid schedule then. out_splits [B] (may be NULL): splits per sequence (0 for a
  * sequence without rows). */
 typedef struct kyro_attention_plan {
     int32_t grid;          /* persistent workgroups */

@@ -988,7 +988,9 @@ int kyro_paged_attention_plan(const kyro_paged_attention_params* p, int num_cus,
         if (num_cus <= 0) num_cus = kDefaultCUs;
         if (chunk_quarters <= 0) chunk_quarters = kyro::kPlanChunkQuarters;
         AttnSetup s;
-        if (int rc = attention_setup(p, q_lens != nullptr, num_cus, s, chunk_quarters)) return rc;
+        // The balanced schedule's answer, also where automatic choice takes short chunks or the
+        // many-row kernel instead.
+        if (int rc = attention_setup(p, q_lens != nullptr, num_cus, s, chunk_quarters, FORMS_LEAST_SCRATCH)) return rc;
         const kyro::AttnArgs& a = s.a;
         if (s.empty) return KYRO_OK;
         if (!context_lens) return fail(KYRO_EINVAL, "paged_attention_plan: context_lens is null");

@@ -135,3 +135,13 @@ def test_grid_schedule_params_are_refused():
 
     with pytest.raises(KyroError, match="grid schedule"):
         attention_plan(PagedAttention(16, 8, 128, 2), [100, 200], None, max_blocks_per_seq=16, schedule="grid")
+
+
+@pytest.mark.parametrize("q,ctx,blocks", [(512, 4000, 256), (1, 1000, 63)])
+def test_plan_answers_where_automatic_choice_takes_another_form(q, ctx, blocks):
+    """A prompt chunk runs on the many-row kernel and a lone decode in short chunks; their balanced plan is
+    still what the schedule by name would run."""
+    attn = PagedAttention(16, 32, 128, 8)
+    kw = dict(q_lens=[q], max_blocks_per_seq=blocks, num_blocks=blocks)
+    auto, by_name = (attention_plan(attn, [ctx], schedule=s, **kw) for s in ("auto", "balanced"))
+    assert auto[0] == by_name[0] and np.array_equal(auto[1], by_name[1])
